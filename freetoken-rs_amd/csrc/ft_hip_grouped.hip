@@ -12,6 +12,8 @@
 //                     in registers, dots against every token of the expert,
 //                     GELU*up, q8 of the act block -> act[pair][j]
 //   k_grouped_down    per (active expert, 128-row unit): y[pair][rows]
+//   k_mfma_gu_tok, k_mfma_down_tok, k_mfma_down  the same two on the int8
+//                     matrix cores, for batches of several tokens per expert
 //   k_grouped_combine x_out[t] = x[t] + sum_k y[t*K+k] * w[t*K+k] in slot order
 // Weights are in the fused layout (ft_hip_pack_experts_fused), so one packed
 // bank serves this path and the batch-1 fused kernel.
@@ -33,6 +35,7 @@ constexpr int NT = 8;         // tokens per chunk of the gate|up kernel (LDS sta
 constexpr int NTD = 16;       // tokens per chunk of the down kernel
 constexpr int DU = 16 * GW;   // rows per down unit (one 16-row tile per wave)
 constexpr int MAX_PAIRS = 4096;
+constexpr int MT = 16;        // tokens per MFMA tile
 
 struct GroupWs {
     float* logits;      // [B][E]
@@ -92,13 +95,21 @@ __device__ __forceinline__ void stage(int n, Ld ld, St st) {
 // to the pair's own slot, so results are the same for any order.
 // Groups are numbered with the experts of >= n_mfma tokens first (meta[1 +
 // 3E] of them, for the MFMA kernels), then the others (for the dot4
-// kernels), each in expert order.
+// kernels), each in expert order. The MFMA groups' token tiles (up to
+// MT tokens of one group each) are listed in ppos[0..P) as tile_entry
+// words.
 //
 // TOPK (E <= 32 as launched): the routing itself first, from the logits (the
 // arithmetic of k_topk_router, so the same ids and weights): 1024/E tokens
 // per round, one thread per logit ranking it by rank_key among its token's
 // E, then the softmax over each token's K in rank order; ids/wts written to
 // ids_out/wts_out and kept in LDS for the grouping.
+// A token tile: the number of tiles (up to 4096: 13 bits, in every entry), its
+// group (10 bits) and its first token / MT (8 bits).
+__host__ __device__ __forceinline__ uint32_t tile_entry(int n_tiles, int g, int c0) {
+    return (uint32_t)n_tiles << 18 | (uint32_t)g << 8 | (uint32_t)c0 / MT;
+}
+
 template <bool TOPK>
 __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P, int E, int n_mfma, int32_t* meta,
                                                       int32_t* plist, int32_t* ppos, const float* logits,
@@ -171,28 +182,35 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
     // totals of the wavefronts before its own (integer sums: exact in any order)
     const int c = t < E ? cnt[t] : 0;
     int vc = c, va = c > 0, vf = c > 0 && c >= n_mfma;
+    const int my_tiles = vf ? (c + MT - 1) / MT : 0;
+    int vt = my_tiles;
     const int lane = t & 63, wv = t >> 6;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const int nc = __shfl_up(vc, d), na = __shfl_up(va, d), nf = __shfl_up(vf, d);
+        const int nc = __shfl_up(vc, d), na = __shfl_up(va, d), nf = __shfl_up(vf, d), ntl = __shfl_up(vt, d);
         if (lane >= d) {
             vc += nc;
             va += na;
             vf += nf;
+            vt += ntl;
         }
     }
-    __shared__ int wtot[3][16];
+    __shared__ int wtot[4][16];
+    __shared__ int n_tiles;
     if (lane == 63) {
         wtot[0][wv] = vc;
         wtot[1][wv] = va;
         wtot[2][wv] = vf;
+        wtot[3][wv] = vt;
     }
     __syncthreads();
     for (int q = 0; q < wv; ++q) {
         vc += wtot[0][q];
         va += wtot[1][q];
         vf += wtot[2][q];
+        vt += wtot[3][q];
     }
+    if (t == 1023) n_tiles = vt;
     scan[t] = vc;
     act[t] = va;
     big[t] = vf;
@@ -212,6 +230,9 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
         const int e = min(max(pid(p), 0), E - 1);
         plist[scan[e] - cnt[e] + ppos[p]] = p;
     }
+    __syncthreads();  // ppos is read: it becomes the tile list (every tile holds a pair, so P entries suffice)
+    for (int k = 0; k < my_tiles; ++k) ppos[vt - my_tiles + k] = (int32_t)tile_entry(n_tiles, big[t] - 1, k * MT);
+    if (t == 0 && n_tiles == 0) ppos[0] = 0;
 }
 
 // The pairs p < P routed to expert e (ids[p] == e), ascending, into lst
@@ -487,11 +508,7 @@ __global__ __launch_bounds__(GT, 1) void k_grouped_down(const uint8_t* bank, int
 // then accumulate as acc = fma(float(D), d4 * d8, acc), in block order.
 // ---------------------------------------------------------------------------
 typedef int v4i __attribute__((ext_vector_type(4)));
-constexpr int MT = 16;  // tokens per MFMA tile
-// token stride of the gate|up wave partials in LDS: one more than MT, so the
-// wave-order sums (consecutive lanes: consecutive rows) read distinct banks
-constexpr int MTP = MT + 1;
-static_assert(MT * 10 <= GT, "k_mfma_gu stores a chunk's q8 words with one thread each");
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 struct ActOp {
     long b;    // B operand: q8 words g and 4+g
@@ -548,6 +565,25 @@ __device__ __forceinline__ long nib_op(uint32_t w) {
     return (long)(((uint64_t)((w >> 4) & 0x0F0F0F0Fu) << 32) | (w & 0x0F0F0F0Fu));
 }
 
+// The same, signed: 16 * (q - 8) as bytes (the nibble in the byte's high half,
+// its top bit flipped), so D is 16 times the block dot, the accumulator starts
+// at zero and qsum is not needed. The kernels that use it take d8 / 16, exact,
+// so a product of scales and every sum has the bits it has with the plain dot
+// (short of products below 2^-122, which are subnormal then).
+__device__ __forceinline__ long nib_op16(uint32_t w) {
+    const uint32_t lo = ((w << 4) & 0xF0F0F0F0u) ^ 0x80808080u, hi = (w & 0xF0F0F0F0u) ^ 0x80808080u;
+    return (long)(((uint64_t)hi << 32) | lo);
+}
+
+// d4 * d8 of a 16x16 tile's (row, token) pairs, each rounded once as by
+// v_mul_f32 (subnormals kept), in the lanes and order of the int8 MFMA's
+// results: v_mfma_f32_4x4x1 is 16 outer products of 4 rows and 4 columns, one
+// per lane quad. Lane (lg, li) gives the scale of row 4*lg + li%4 and its
+// token's d. One instruction on the matrix cores (8 cycles) for four VALU ones.
+__device__ __forceinline__ v4f scale_products(float d4, float d8) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(d4, d8, v4f{0, 0, 0, 0}, 0, 0, 0);
+}
+
 __device__ __forceinline__ v4i c_init(int qsum) {
     const int c = -8 * qsum;
     const v4i v = {c, c, c, c};
@@ -563,286 +599,383 @@ __device__ __forceinline__ void scales4(const uint16_t* p, float (&sc)[4]) {
     sc[3] = h2f((uint16_t)(s2.y >> 16));
 }
 
-// Gate|up tiles of the MFMA groups (tile j: 64 rows, gate rows 32j.. and up
-// rows I+32j..), each for its expert's tokens 16 at a time, then GELU*up and
-// the q8 of act block j per token. Persistent: one workgroup per CU walks a
-// contiguous range of (expert group, tile j) items, each in chunks of 16
-// tokens (units). Wave w takes blocks [w*BPW, (w+1)*BPW) of the 64 rows as
-// four 16-row MFMA tiles; the 8 wave partials of a (row, token) are summed
-// in wave order. The tokens' q8 rows of the current chunk sit in LDS
-// (staged when the group or chunk changes, which a contiguous range makes
-// rare), so the MFMA B operands are LDS reads, read one block ahead. The
-// weights stream through registers: a wave holds its BPW blocks' qs dwords
-// of a unit, and consuming block b refills that slot with block b of the
-// NEXT unit, so the next tile streams during this unit's MFMAs and its
-// epilogue (wave sums, GELU*up, q8). A tile's f16 scales go through one LDS
-// buffer as f32 (widened once there, not by each of the 16 lanes of a lane
-// group per block): the next unit's are loaded into registers (16 bytes per
-// thread and round) once every wave is past this unit's MFMAs, and stored to
-// LDS at the end of this unit's epilogue. Per (row, token): acc = fma(float(D_b), d4_b *
-// d8_b, acc) over the wave's blocks in block order, then the wave partials in
-// wave order.
+// Gate|up of the MFMA groups by token tiles: workgroup (x, y) takes act blocks
+// x*NW .. x*NW + NW-1 (one wave each: the 64 rows of tile j) for tile y of the
+// token tiles that k_group_pairs lists (up to 16*TT tokens of one expert).
+// The tokens' q8 rows are staged in LDS once, by block, so that a lane's
+// operand words are one 8-byte read; a wave streams its tile's rows through a
+// register ring of one K slice (BPW blocks, 1 KB per load), its scales
+// through an LDS buffer of its own, and keeps all of a (row, token)'s sums:
+// per slice acc = fma(float(D_b), d4_b * d8_b, acc) in block order, then the 8
+// slice sums in order, the same bits as k_grouped_gu's. A lane holds
+// gate and up of the same columns, so GELU*up and the act block's q8 stay in
+// registers (two lane exchanges for the block's amax and sum), and go out as
+// the q8m words they are.
 //
-// The scales once went to LDS by direct global-to-LDS loads two units ahead.
-// A load into LDS completes in order behind the ring's weight loads, and the
-// compiler cannot tell it apart from the epilogue's LDS traffic: the fence of
-// the next barrier and the next LDS read each waited for it with s_waitcnt
-// vmcnt(0), which drained the next unit's weight loads at the start of every
-// epilogue. Loaded into registers, the only wait is the one before their LDS
-// store at the end of the epilogue.
-
-struct MfUnit {
-    const uint8_t* T;  // the tile: [nb][64] f16 scales, then [nb][64][16 B] qs
-    int g, s0, n, j, c0, nt, item;
-    bool live;
-};
-
-template <int BPW, bool REC>
-__global__ __launch_bounds__(GT, 1) void k_mfma_gu(const uint8_t* __restrict__ bank, int64_t expert_bytes,
-                                                     const int32_t* __restrict__ meta,
-                                                     const int32_t* __restrict__ plist,
-                                                     const uint8_t* __restrict__ q8x, uint8_t* q8m, float* dbg_gu,
-                                                     const float* __restrict__ in_scale, int H, int I, int E, int K,
-                                                     int P, int32_t* rec) {
+// Why this form: the former kernel split K over the 8 waves of a workgroup,
+// summed their partials through LDS for every 16 tokens and restaged the
+// tokens' rows, an integer division and two dependent loads per word, at each
+// tile of a group of over 16 tokens, on ranges of tiles that skewed token
+// counts left uneven: 475 us for 512 tokens of the Gemma shape and 855 us for
+// 173 zipf-skewed ones. Here a wave needs no other wave: 118-126 and 67 us.
+// What bounds it: for many tokens the VALU (72 % busy: 16 conversions and 16
+// fmas per block and wave are left after the scale products moved to the
+// matrix cores, 24 for operands and 10 for the GELU epilogue); for few the
+// weights (64 tokens: 285 MB in 63 us, 4.5 TB/s). Blocks are consumed one at a
+// time (sched_barrier), else the registers of a whole slice's dots spill.
+template <int BPW, int NW, int WPE, int D, int KH, bool REC>
+__global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __restrict__ bank, int64_t expert_bytes,
+                                                         const int32_t* __restrict__ meta,
+                                                         const uint32_t* __restrict__ tiles,
+                                                         const int32_t* __restrict__ plist,
+                                                         const uint8_t* __restrict__ q8x, uint8_t* q8m, float* dbg_gu,
+                                                         const float* __restrict__ in_scale, int I, int E, int K, int P,
+                                                         int32_t* rec) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int SPT = (128 * 128 + GT * 16 - 1) / (GT * 16);  // scale rounds, up to nb = 128 (H 4096)
-    const int nb = H >> 5, nbj = I >> 5;
-    const int n_items = meta[1 + 3 * E] * nbj;  // (group, tile) pairs of the MFMA groups (first in the list)
-    const int per = (n_items + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int it0 = (int)blockIdx.x * per, it1 = min(n_items, it0 + per);
-    if (it0 >= it1) return;
-    // LDS: scales [nb][64] f32 | wave partials [GW][64][MTP] | sums [MT][64] |
-    // act [MT][32] | act q8 [MT][10] | the chunk's tokens (pair, norm scale)
-    // [MT] x2 | the chunk's q8 rows [MT][nb*10 + 1] u32
-    float* scl = reinterpret_cast<float*>(lds);
-    float* red = reinterpret_cast<float*>(lds + nb * 256);
-    float* rows = red + GW * 64 * MTP;
-    float* actv = rows + MT * 64;
-    uint32_t* ablk = reinterpret_cast<uint32_t*>(actv + MT * 32);
-    int* tok_p = reinterpret_cast<int*>(ablk + MT * 10);
-    float* tok_s = reinterpret_cast<float*>(tok_p + MT);
-    uint32_t* xq = reinterpret_cast<uint32_t*>(tok_s + MT);
-    const int xs = nb * 10 + 1;  // token stride (dwords), odd: the 16 tokens' rows start in different banks
-    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), li = t & 15, lg = (t >> 4) & 3;
-    const int b0 = wave * BPW;
-    const uint32_t vw16 = lg * 256 + li * 16;
-    auto bind = [&](int it, int c, bool live) __attribute__((always_inline)) {
-        MfUnit u;
-        u.live = live;
-        u.item = it;
-        it = live ? it : it0;  // a dead unit is bound to a valid item and never computed
-        u.g = it / nbj;
-        u.j = it - u.g * nbj;
-        const int e = meta[1 + u.g];
-        u.s0 = meta[1 + E + u.g];
-        u.n = meta[1 + 2 * E + u.g];
-        u.c0 = live ? c : 0;
-        u.nt = min(MT, u.n - u.c0);
-        u.T = bank + (int64_t)e * expert_bytes + (int64_t)u.j * nb * 1152;
-        return u;
-    };
-    auto after = [&](const MfUnit& u) __attribute__((always_inline)) {  // the unit after u in this range
-        if (!u.live) return u;
-        if (u.c0 + MT < u.n) return bind(u.item, u.c0 + MT, true);
-        return bind(u.item + 1, 0, u.item + 1 < it1);
-    };
-    auto same_tile = [](const MfUnit& a, const MfUnit& c) { return a.g == c.g && a.j == c.j; };
-    uint32_t aw[BPW][4];
-    // slot b <- block b of unit u (dead: a descriptor of 0 bytes returns zeros and reads nothing)
-    auto issue_block = [&](int b, const MfUnit& u) __attribute__((always_inline)) {
-        // one 16-byte load: lane group g takes the four qs words of row
-        // 16g + li (1 KB contiguous per wave); quad_transpose turns them into
-        // word g of rows li, 16 + li, 32 + li, 48 + li when the block is used
-        const __amdgpu_buffer_rsrc_t rw = buf_rsrc(u.T + nb * 128, u.live ? (uint32_t)nb * 1024 : 0u);
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, (b0 + b) * 1024, 0);
-        aw[b][0] = v.x;
-        aw[b][1] = v.y;
-        aw[b][2] = v.z;
-        aw[b][3] = v.w;
-    };
-    // unit u's tile scales (nb * 128 bytes of f16) into registers, 16 bytes
-    // per thread and round (dead or past the end: zeros, nothing read), and
-    // from there, widened, into scl once no wave reads the previous tile's
-    u32x4 sst[SPT];
-    auto load_scales = [&](const MfUnit& u) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(u.T, u.live ? (uint32_t)nb * 128 : 0u);
+    constexpr int NB = 8 * BPW, TM = MT, NTH = NW * 64;
+    constexpr int XS = TM * 8 + 2;  // words per block of the qs: a pad of two, so that lanes on consecutive blocks write distinct banks
+    constexpr int NH = NB / KH, SH = 8 / KH;  // blocks and slices per staging of the tokens' rows
+    constexpr int R = (TM * NH + NTH - 1) / NTH;  // (token, block) items staged per thread
+    constexpr int SW = BPW * 128;   // bytes of a slice's scales
+    const int nbj = I >> 5, JG = (nbj + NW - 1) / NW;
+    // workgroup id % 8 is the XCD: each takes a contiguous eighth of the (tile, act block group) units, so
+    // the tiles of one expert, which read the same weights, run together behind one L2
+    const int n_units = (int)(tiles[0] >> 18) * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
+    const int unit = ((int)blockIdx.x & 7) * per + ur;
+    if (ur >= per || unit >= n_units) return;
+    const uint32_t v0 = tiles[unit / JG];
+    const int jg = unit % JG, g = (int)(v0 >> 8) & 1023, c0 = (int)(v0 & 255) * MT;
+    const int e = meta[1 + g], s0 = meta[1 + E + g], nt = min(TM, meta[1 + 2 * E + g] - c0);
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
+    const int jw = jg * NW + wave, j = min(jw, nbj - 1);
+    // LDS: the tokens' q8 words [NH][4 lane groups][TM] (g, g+4) | [NH][TM] d / 16 | the waves' slice scales
+    uint32_t* xq = reinterpret_cast<uint32_t*>(lds);
+    float* xd = reinterpret_cast<float*>(lds + (size_t)NH * XS * 4);
+    uint8_t* scl = lds + (size_t)NH * (XS * 4 + TM * 4) + wave * SW;
+    // the tokens' rows: thread item i = (token, block), 40 bytes
+    uint2 st[R][5];
+    auto load_act = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < SPT; ++r)  // the offset in the per-lane part: that is the part the range check sees
-            sst[r] = __builtin_amdgcn_raw_buffer_load_b128(rs, (r * GT + t) * 16, 0, 0);
-    };
-    auto store_scales = [&]() __attribute__((always_inline)) {
+        for (int r = 0; r < R; ++r) {
+            const int i = r * NTH + t, tt = i / NH, b = i - tt * NH;
+            if (tt < nt) {
+                const uint2* src =
+                    reinterpret_cast<const uint2*>(q8x + ((int64_t)(plist[s0 + c0 + tt] / K) * NB + h * NH + b) * Q8_BLK);
 #pragma unroll
-        for (int r = 0; r < SPT; ++r) {
-            const int i = (r * GT + t) * 8;  // the first of this thread's 8 scales
-            if (i < nb * 64) {
-                const u32x4 h = sst[r];
-                float4* d = reinterpret_cast<float4*>(scl + i);
-                d[0] = make_float4(h2f((uint16_t)(h.x & 0xFFFF)), h2f((uint16_t)(h.x >> 16)),
-                                   h2f((uint16_t)(h.y & 0xFFFF)), h2f((uint16_t)(h.y >> 16)));
-                d[1] = make_float4(h2f((uint16_t)(h.z & 0xFFFF)), h2f((uint16_t)(h.z >> 16)),
-                                   h2f((uint16_t)(h.w & 0xFFFF)), h2f((uint16_t)(h.w >> 16)));
+                for (int k = 0; k < 5; ++k) st[r][k] = src[k];
             }
         }
     };
-    // unit u's tokens (pair, norm scale) into tok_p/tok_s and their q8 rows
-    // into xq (token slots >= nt: the last token again; their MFMA columns
-    // are never read). Only between units; the caller syncs afterwards.
-    auto stage_act = [&](const MfUnit& u) __attribute__((always_inline)) {
-        if (t < MT) {
-            const int pp = plist[u.s0 + u.c0 + min(t, u.nt - 1)];
-            tok_p[t] = pp;
-            tok_s[t] = in_scale ? in_scale[pp / K] : 1.0f;
-        }
-        __syncthreads();
-        const int per_tok = nb * 10;
-        for (int i = t; i < MT * per_tok; i += GT) {
-            const int tt = i / per_tok, w = i - tt * per_tok;
-            xq[tt * xs + w] = reinterpret_cast<const uint32_t*>(q8x + (int64_t)(tok_p[tt] / K) * nb * Q8_BLK)[w];
-        }
-    };
-    // a block's LDS operands: this lane's token words, its d and qsum, and
-    // the scales of rows 16m + 4lg .. +3 for the 4 tiles m
-    struct Ops {
-        uint32_t lo, hi, d, qsum;
-        float4 sc[4];
-    };
-    MfUnit cur = bind(it0, 0, true);
-    MfUnit nxt = after(cur);
-    load_scales(cur);
+    auto store_act = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < BPW; ++b) issue_block(b, cur);
-    store_scales();
-    stage_act(cur);
-    int act_g = cur.g, act_c0 = cur.c0;  // the chunk whose q8 rows are in xq
+        for (int r = 0; r < R; ++r) {
+            const int i = r * NTH + t, tt = i / NH, b = i - tt * NH;
+            if (tt < nt) {
+                uint32_t* q = xq + b * XS + tt * 2;
+                *reinterpret_cast<uint2*>(q) = make_uint2(st[r][1].x, st[r][3].x);
+                *reinterpret_cast<uint2*>(q + TM * 2) = make_uint2(st[r][1].y, st[r][3].y);
+                *reinterpret_cast<uint2*>(q + TM * 4) = make_uint2(st[r][2].x, st[r][4].x);
+                *reinterpret_cast<uint2*>(q + TM * 6) = make_uint2(st[r][2].y, st[r][4].y);
+                xd[b * TM + tt] = __uint_as_float(st[r][0].x) * 0.0625f;
+            }
+        }
+    };
+    load_act(0);
+    const uint8_t* T = bank + (int64_t)e * expert_bytes + (int64_t)j * NB * 1152;
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(T, NB * 128), rw = buf_rsrc(T + NB * 128, NB * 1024);
+    const uint32_t vw16 = lg * 256 + li * 16;
+    u32x4 aw[BPW], ss[2];
+    auto load_scales = [&](int s) __attribute__((always_inline)) {  // the slice's scales, 16 bytes a lane and round
+        ss[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, s * SW, 0);
+        ss[1] = __builtin_amdgcn_raw_buffer_load_b128(rs, min(1024 + lane * 16, SW - 16), s * SW, 0);
+    };
+    load_scales(0);
+#pragma unroll
+    for (int b = 0; b < D; ++b) aw[b] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, b * 1024, 0);
+    store_act();
     __syncthreads();
-    auto step = [&]() __attribute__((always_inline)) {
-        const MfUnit n2 = after(nxt);
-        const bool nxt_scales = nxt.live && !same_tile(nxt, cur);  // a new tile (else scl already holds them)
-        const int pme = tok_p[li];  // this lane's token pair (REC)
-        const uint32_t* xl = xq + li * xs;  // this lane's token row
-        auto ops = [&](int blk) __attribute__((always_inline)) {
-            Ops o;
-            o.lo = xl[blk * 10 + 2 + lg];
-            o.hi = xl[blk * 10 + 6 + lg];
-            o.d = xl[blk * 10];
-            o.qsum = xl[blk * 10 + 1];
+    if (KH == 1 && jw >= nbj) return;
+    const int slot = min(li, nt - 1);  // this lane's token (past the end: the last one, never written)
+    float tot[4][4];                   // [row tile][row]
 #pragma unroll
-            for (int m = 0; m < 4; ++m) o.sc[m] = *reinterpret_cast<const float4*>(scl + blk * 64 + 16 * m + 4 * lg);
-            return o;
-        };
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tot[m][v] = 0.0f;
+    auto slice = [&](int s, auto lastt) __attribute__((always_inline)) {
+        constexpr bool last = decltype(lastt)::value;
+        // the slice's scales into this wave's buffer (its reads of the slice before have all returned)
+        asm volatile("" ::: "memory");
+        *reinterpret_cast<u32x4*>(scl + lane * 16) = ss[0];
+        if (1024 + lane * 16 < SW) *reinterpret_cast<u32x4*>(scl + 1024 + lane * 16) = ss[1];
+        asm volatile("" ::: "memory");
+        if (!last) load_scales(s + 1);
         float acc[4][4];
 #pragma unroll
         for (int m = 0; m < 4; ++m)
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[m][v] = 0.0f;
-        Ops o = ops(b0);
 #pragma unroll
         for (int b = 0; b < BPW; ++b) {
-            const int blk = b0 + b;
-            const Ops cu = o;
-            if (b + 1 < BPW) o = ops(blk + 1);  // the next block's LDS operands, in flight during these MFMAs
-            const v4i c = c_init((int)cu.qsum);
-            const long bop = (long)(((uint64_t)cu.hi << 32) | cu.lo);
-            v4i d[4];
-            quad_transpose(aw[b][0], aw[b][1], aw[b][2], aw[b][3]);
+            const int blk = s % SH * BPW + b;
+            const uint2 q = *reinterpret_cast<const uint2*>(xq + blk * XS + (lg * TM + slot) * 2);
+            const float ad = xd[blk * TM + slot];
+            float dw[4];
 #pragma unroll
-            for (int m = 0; m < 4; ++m) d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op(aw[b][m]), bop, c, 0, 0, 0);
-            issue_block(b, nxt);
-            const float ad = __uint_as_float(cu.d);
+            for (int m = 0; m < 4; ++m)
+                dw[m] = h2f(*reinterpret_cast<const uint16_t*>(scl + b * 128 + m * 32 + lg * 8 + (li & 3) * 2));
+            uint32_t w[4] = {aw[b].x, aw[b].y, aw[b].z, aw[b].w};
+            quad_transpose(w[0], w[1], w[2], w[3]);
+            if (b + D < BPW || !last)  // the block D ahead
+                aw[(b + D) % BPW] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, (s * BPW + b + D) * 1024, 0);
+            const long bop = (long)(((uint64_t)q.y << 32) | q.x);
+            v4i d[4];
+            v4f sp[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) sp[m] = scale_products(dw[m], ad);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op16(w[m]), bop, v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
-                if constexpr (REC) {  // test record: D = the (row, token) blocks' int32 dots
-                    if (li < cur.nt)
+                if constexpr (REC) {  // test record: the (row, token) blocks' int32 dots
+                    if (li < nt && jw < nbj)
 #pragma unroll
                         for (int v = 0; v < 4; ++v) {
                             const int rr = 16 * m + 4 * lg + v;
-                            const int row = rr < 32 ? cur.j * 32 + rr : I + cur.j * 32 + (rr - 32);
-                            rec[((int64_t)pme * 2 * I + row) * nb + blk] = d[m][v];
+                            const int row = rr < 32 ? j * 32 + rr : I + j * 32 + (rr - 32);
+                            rec[((int64_t)plist[s0 + c0 + slot] * 2 * I + row) * NB + s * BPW + b] = d[m][v] >> 4;
                         }
                 }
-                const float sc[4] = {cu.sc[m].x, cu.sc[m].y, cu.sc[m].z, cu.sc[m].w};
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[m][v] = fmaf((float)d[m][v], sc[v] * ad, acc[m][v]);
+                for (int v = 0; v < 4; ++v) acc[m][v] = fmaf((float)d[m][v], sp[m][v], acc[m][v]);
+                // the sums are formed here: left to the scheduler, the dots of a whole slice wait for theirs
+                asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
             }
             __builtin_amdgcn_sched_barrier(0);  // one block's MFMA results live at a time
         }
 #pragma unroll
         for (int m = 0; m < 4; ++m)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) red[(wave * 64 + 16 * m + 4 * lg + v) * MTP + li] = acc[m][v];
-        __syncthreads();  // every wave is past its MFMAs: act rows and scl may change below
-        if (nxt_scales) load_scales(nxt);
-        for (int i = t; i < cur.nt * 64; i += GT) {  // (token, row) sums over the waves, in wave order
-            const int tt = i >> 6, rr = i & 63;
-            float sv = 0.0f;
-#pragma unroll
-            for (int v = 0; v < GW; ++v) sv = sv + red[(v * 64 + rr) * MTP + tt];
-            const int pp = tok_p[tt];
-            if (in_scale) sv = sv * tok_s[tt];
-            rows[tt * 64 + rr] = sv;
-            if (dbg_gu) dbg_gu[(int64_t)pp * 2 * I + (rr < 32 ? cur.j * 32 + rr : I + cur.j * 32 + (rr - 32))] = sv;
-        }
-        __syncthreads();
-        for (int i = t; i < cur.nt * 32; i += GT) {
-            const int tt = i >> 5, cc = i & 31;
-            actv[tt * 32 + cc] = gelu_tanh(rows[tt * 64 + cc]) * rows[tt * 64 + 32 + cc];
-        }
-        __syncthreads();
-        if (t < 4 * cur.nt) quantize_block_quad(actv + (t >> 2) * 32, t & 3, ablk + (t >> 2) * 10);
-        __syncthreads();
-        if (t < cur.nt * 10) {  // q8m at group position q (MT * 10 <= GT)
-            const int tt = t / 10, wd = t - tt * 10, q = cur.s0 + cur.c0 + tt, wq = wd - 2;
-            const uint32_t o = wd < 2 ? (uint32_t)((P * nbj * 4 + cur.j * P + q) * 2 + wd)
-                                      : (uint32_t)(((cur.j * 4 + (wq & 3)) * P + q) * 2 + (wq >> 2));
-            reinterpret_cast<uint32_t*>(q8m)[o] = ablk[t];
-        }
-        if (!nxt.live) return false;
-        if (nxt_scales) store_scales();
-        if (nxt.g != act_g || nxt.c0 != act_c0) {
-            stage_act(nxt);
-            act_g = nxt.g;
-            act_c0 = nxt.c0;
-        }
-        __syncthreads();
-        cur = nxt;
-        nxt = n2;
-        return true;
+            for (int v = 0; v < 4; ++v) tot[m][v] = tot[m][v] + acc[m][v];
     };
-    while (step()) {
+#pragma unroll 1
+    for (int s = 0; s < 7; ++s) {
+        if (KH > 1 && s == SH) {  // the rest of the tokens' rows, once every wave is done with the first part
+            load_act(1);
+            __syncthreads();
+            store_act();
+            __syncthreads();
+        }
+        slice(s, std::false_type{});
+    }
+    slice(7, std::true_type{});
+    if (KH > 1 && jw >= nbj) return;
+    const int q = s0 + c0 + slot, p = plist[q];
+    const bool ok = li < nt;
+    const float isc = in_scale ? in_scale[p / K] : 1.0f;
+    float a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // columns 16*(i/4) + 4*lg + i%4 of the act block
+        float gv = tot[i >> 2][i & 3], uv = tot[2 + (i >> 2)][i & 3];
+        if (in_scale) {
+            gv = gv * isc;
+            uv = uv * isc;
+        }
+        if (dbg_gu && ok) {
+            const int64_t o = (int64_t)p * 2 * I + j * 32 + (i >> 2) * 16 + lg * 4 + (i & 3);
+            dbg_gu[o] = gv;
+            dbg_gu[o + I] = uv;
+        }
+        a[i] = gelu_tanh(gv) * uv;
+        __builtin_amdgcn_sched_barrier(0);  // one GELU's registers at a time
+    }
+    // the block's q8 over its four lanes (li + 16*lg), the arithmetic of quantize_block_quad
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(a[i]));
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    const float d = amax > 0.0f ? amax / 127.0f : 0.0f;
+    const float inv = d > 0.0f ? 1.0f / d : 0.0f;
+    int qsum = 0;
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int qi = (int)q8_clamp(roundf(a[i] * inv));
+        qsum += qi;
+        w[i >> 2] |= (uint32_t)(uint8_t)(int8_t)qi << (8 * (i & 3));
+    }
+    qsum += __shfl_xor(qsum, 16);
+    qsum += __shfl_xor(qsum, 32);
+    if (ok) {
+        uint2* o = reinterpret_cast<uint2*>(q8m);
+        o[(uint32_t)((j * 4 + lg) * P + q)] = make_uint2(w[0], w[1]);
+        if (lg == 0) o[(uint32_t)(P * nbj * 4 + j * P + q)] = make_uint2(__float_as_uint(d), (uint32_t)qsum);
     }
 }
 
-// Down rows of active expert g for its tokens, 16 at a time. The workgroup
-// takes GW/KS groups of RT consecutive 16-row down tiles; wave w works on the
-// RT tiles of group w/KS (they share each block's activation operand), K
-// slice w%KS (blocks [s*BW, s*BW+BW) below nbj); the KS slice partials of a
-// (row, token) are summed in slice order into y[pair][row]. With KS > 1 the
-// partials overlay the tiles' scales in LDS (restaged for each 16 tokens),
-// so two workgroups fit a CU. Blocks go in NBB-block batches, NBUF batches in
+// Down rows by token tiles, for rows of up to 4*NKB blocks: a wave takes 64
+// rows (four 16-row tiles) of one expert for the up to 16 tokens of one token
+// tile, workgroup unit (tile, NW waves of rows). The tokens' act words come
+// from q8m as they lie (each block's words of a lane group contiguous over the
+// group's tokens) and are staged in LDS once for the workgroup's waves; the
+// rows stream through registers four blocks (NBUF - 1 batches) ahead. Per
+// (row, token) acc = fma(float(D_b), d4_b * d8_b, acc) in block order. Four
+// waves of about 94 registers per workgroup, several to a CU, so that one's
+// staging runs under another's dots (8 waves 64 us against 57 at 512 tokens;
+// two batches ahead instead of one 58.5). Before, one workgroup walked all of
+// an expert's tokens, rereading the weights for each 16: 512 tokens of the
+// Gemma shape 104 us, 173 zipf-skewed 93, 64 tokens 47; now 57, 31 and 33
+// (143 MB of weights, 4.4 TB/s).
+template <int NKB, int NBUF, int NW, bool REC>
+__global__ __launch_bounds__(NW * 64, 4) void k_mfma_down_tok(const uint8_t* __restrict__ bank, int64_t expert_bytes,
+                                                               int64_t gu_bytes, const int32_t* __restrict__ meta,
+                                                               const uint32_t* __restrict__ tiles,
+                                                               const int32_t* __restrict__ plist,
+                                                               const uint8_t* __restrict__ q8m, int P, float* ydn, int H,
+                                                               int I, int E, int32_t* rec) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    constexpr int NTH = NW * 64;
+    const int nbj = I >> 5, dn_tile = nbj * 288, RG = H / 64, JG = (RG + NW - 1) / NW;
+    const int n_units = (int)(tiles[0] >> 18) * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
+    const int unit = ((int)blockIdx.x & 7) * per + ur;  // as k_mfma_gu_tok's
+    if (ur >= per || unit >= n_units) return;
+    const uint32_t v0 = tiles[unit / JG];
+    const int g = (int)(v0 >> 8) & 1023, c0 = (int)(v0 & 255) * MT;
+    const int e = meta[1 + g], s0 = meta[1 + E + g], nt = min(MT, meta[1 + 2 * E + g] - c0);
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
+    const int rw0 = (unit % JG) * NW + wave, rg = min(rw0, RG - 1);  // this wave's 64 rows
+    // LDS: the tokens' act words [nbj][4][MT] (g, g+4) | [nbj][MT] d / 16 | the waves' scales [4][nbj][16] f16
+    uint2* xq = reinterpret_cast<uint2*>(lds);
+    float* xd = reinterpret_cast<float*>(lds + (size_t)nbj * 512);
+    uint8_t* scl = lds + (size_t)nbj * 576 + (size_t)wave * nbj * 128;
+    const __amdgpu_buffer_rsrc_t rw =
+        buf_rsrc(bank + (int64_t)e * expert_bytes + gu_bytes + (int64_t)rg * 4 * dn_tile, (uint32_t)(4 * dn_tile));
+    u32x4 ss[4], aw[NBUF][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        ss[m] = __builtin_amdgcn_raw_buffer_load_b128(rw, min(lane * 16, nbj * 32 - 16), m * dn_tile, 0);
+    auto load = [&](int kb, int buf) __attribute__((always_inline)) {  // lane group g: block 4*kb + g of row li of each tile
+        const uint32_t vo = nbj * 32 + min(4 * kb + lg, nbj - 1) * 256 + li * 16;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) aw[buf][m] = __builtin_amdgcn_raw_buffer_load_b128(rw, vo, m * dn_tile, 0);
+    };
+#pragma unroll
+    for (int k = 0; k < NBUF - 1; ++k) load(k, k);
+    {
+        constexpr int R = (4 * NKB * 64 + NTH - 1) / NTH, RD = (4 * NKB * 16 + NTH - 1) / NTH;
+        const uint2* q2 = reinterpret_cast<const uint2*>(q8m);
+        uint2 w[R];
+        float dv[RD];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {  // slots past the tile: the last token again, never written out
+            const int i = r * NTH + t, tt = min(i & 15, nt - 1);
+            if (i < nbj * 64) w[r] = q2[(int64_t)(i >> 4) * P + s0 + c0 + tt];
+        }
+#pragma unroll
+        for (int r = 0; r < RD; ++r) {
+            const int i = r * NTH + t, tt = min(i & 15, nt - 1);
+            if (i < nbj * 16) dv[r] = __uint_as_float(q2[(int64_t)P * nbj * 4 + (int64_t)(i >> 4) * P + s0 + c0 + tt].x) * 0.0625f;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (r * NTH + t < nbj * 64) xq[r * NTH + t] = w[r];
+#pragma unroll
+        for (int r = 0; r < RD; ++r)
+            if (r * NTH + t < nbj * 16) xd[r * NTH + t] = dv[r];
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        if (lane * 16 < nbj * 32) *reinterpret_cast<u32x4*>(scl + m * nbj * 32 + lane * 16) = ss[m];
+    __syncthreads();
+    if (rw0 >= RG) return;
+    float acc[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[m][v] = 0.0f;
+    const int p = plist[s0 + c0 + min(li, nt - 1)];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+        if (kb + NBUF - 1 < NKB) load(kb + NBUF - 1, (kb + NBUF - 1) % NBUF);
+        uint32_t w[4][4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const u32x4 v = aw[kb % NBUF][m];
+            w[m][0] = v.x;
+            w[m][1] = v.y;
+            w[m][2] = v.z;
+            w[m][3] = v.w;
+            quad_transpose(w[m][0], w[m][1], w[m][2], w[m][3]);
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int blk = kb * 4 + b;
+            if (blk < nbj) {  // uniform
+                const uint2 q = xq[(blk * 4 + lg) * MT + li];
+                const float ad = xd[blk * MT + li];
+                const long bop = (long)(((uint64_t)q.y << 32) | q.x);
+                v4i d[4];
+                v4f sp[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const float dw = h2f(*reinterpret_cast<const uint16_t*>(scl + (m * nbj + blk) * 32 + lg * 8 + (li & 3) * 2));
+                    sp[m] = scale_products(dw, ad);
+                }
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op16(w[m][b]), bop, v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    if constexpr (REC) {  // test record: the (row, token) blocks' int32 dots
+                        if (li < nt)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                rec[((int64_t)p * H + rg * 64 + m * 16 + 4 * lg + v) * nbj + blk] = d[m][v] >> 4;
+                    }
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[m][v] = fmaf((float)d[m][v], sp[m][v], acc[m][v]);
+                    asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // one block's MFMA results live at a time
+        }
+    }
+    if (li < nt) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            *reinterpret_cast<float4*>(ydn + (int64_t)p * H + rg * 64 + m * 16 + 4 * lg) =
+                make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
+    }
+}
+
+// Down rows of over 32 blocks of active expert g for its tokens, 16 at a time.
+// The workgroup takes RT consecutive 16-row down tiles (they share each
+// block's activation operand); wave w works on K slice w (blocks [w*BW,
+// w*BW+BW) below nbj); the slice partials of a (row, token) are summed in
+// slice order into y[pair][row]. The partials overlay the tiles' scales in LDS
+// (restaged for each 16 tokens), so two workgroups fit a CU. Blocks go in NBB-block batches, NBUF batches in
 // flight (register buffers).
-template <int KS, int BW, int RT, int NBB, int NBUF, bool REC>
+template <int BW, int RT, int NBB, int NBUF, bool REC>
 __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_t expert_bytes, int64_t gu_bytes,
                                                      const int32_t* meta, const int32_t* plist, const uint8_t* q8m,
                                                      int P, float* ydn, int H, int I, int E, int n_min,
                                                      int32_t* rec) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int TPW = GW / KS;   // tile groups per workgroup
-    constexpr int TW = TPW * RT;   // tiles per workgroup
     const int nbj = I >> 5, dn_tile = nbj * 288;
     const int u = blockIdx.x, g = blockIdx.y;
     if (g >= meta[1 + 3 * E]) return;  // groups of >= n_min tokens come first
     const int e = meta[1 + g], s0 = meta[1 + E + g], n = meta[1 + 2 * E + g];
     if (n < n_min) return;
-    // LDS: the tiles' scales [TW][nbj][16] f16; slice partials [GW][RT][16][MT]
+    // LDS: the tiles' scales [RT][nbj][16] f16; slice partials [GW][RT][16][MT]
     // in the same bytes once the K loop is done
     uint16_t* scl = reinterpret_cast<uint16_t*>(lds);
     float* red = reinterpret_cast<float*>(lds);
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), li = t & 15, lg = (t >> 4) & 3;
-    const int tl = wave / KS, sl = wave % KS, bs = sl * BW;
-    const int tile0 = (u * TPW + tl) * RT;  // this wave's first tile
+    const int bs = wave * BW;
+    const int tile0 = u * RT;
     const uint8_t* D0 = bank + (int64_t)e * expert_bytes + gu_bytes;  // the expert's down tiles
-    const uint16_t* st = scl + tl * RT * nbj * 16;
-    // the wave's RT tiles: qs of tile tile0+m at m*dn_tile + nbj*32 from D0 + tile0*dn_tile
+    // the RT tiles: qs of tile tile0+m at m*dn_tile + nbj*32 from D0 + tile0*dn_tile
     const __amdgpu_buffer_rsrc_t rw = buf_rsrc(D0 + (int64_t)tile0 * dn_tile, (uint32_t)(RT * dn_tile));
     const __amdgpu_buffer_rsrc_t ra = buf_rsrc(q8m, (uint32_t)P * nbj * Q8_BLK);  // < NO_TOKEN bytes
     const uint32_t vw = nbj * 32 + li * 16 + 4 * lg, vw4 = nbj * 32 + lg * 256 + li * 16;
@@ -896,16 +1029,14 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
 #pragma unroll
         for (int k = 0; k < NBUF - 1; ++k)
             if (k < nbat) load(k, k);
-        if (c0 == 0 || KS > 1) {  // the tiles' scales to LDS, with the first batches in flight
-            stage<8>(
-                TW * nbj * 8,
-                [&](int i) {
-                    const int k = i / (nbj * 8), r = i - k * nbj * 8;
-                    return reinterpret_cast<const uint32_t*>(D0 + (int64_t)(u * TW + k) * dn_tile)[r];
-                },
-                [&](int i, uint32_t v) { reinterpret_cast<uint32_t*>(scl)[i] = v; });
-            __syncthreads();
-        }
+        stage<8>(  // the tiles' scales to LDS, with the first batches in flight
+            RT * nbj * 8,
+            [&](int i) {
+                const int k = i / (nbj * 8), r = i - k * nbj * 8;
+                return reinterpret_cast<const uint32_t*>(D0 + (int64_t)(tile0 + k) * dn_tile)[r];
+            },
+            [&](int i, uint32_t v) { reinterpret_cast<uint32_t*>(scl)[i] = v; });
+        __syncthreads();
         // rounds of NBUF batches, register buffer j holding batch kb + j; the
         // rounds are a loop (not unrolled), so a block's offsets are scalar
         // adds rather than registers held across the slice
@@ -938,7 +1069,7 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
                                     rec[((int64_t)p * H + (tile0 + m) * 16 + 4 * lg + v) * nbj + bs + k * NBB + b] = d[v];
                         }
                         float sc[4];
-                        scales4(st + (m * nbj + bs + k * NBB + b) * 16 + 4 * lg, sc);
+                        scales4(scl + (m * nbj + bs + k * NBB + b) * 16 + 4 * lg, sc);
 #pragma unroll
                         for (int v = 0; v < 4; ++v) acc[m][v] = fmaf((float)d[v], sc[v] * a.d, acc[m][v]);
                     }
@@ -947,30 +1078,20 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
             }
           }
         }
-        if (KS == 1) {
-            if (li < nt) {
+        __syncthreads();  // every wave is done with the scales
 #pragma unroll
-                for (int m = 0; m < RT; ++m)
+        for (int m = 0; m < RT; ++m)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) ydn[(int64_t)p * H + (tile0 + m) * 16 + 4 * lg + v] = acc[m][v];
-            }
-        } else {
-            __syncthreads();  // every wave is done with the scales
+            for (int v = 0; v < 4; ++v) red[((wave * RT + m) * 16 + 4 * lg + v) * MT + li] = acc[m][v];
+        __syncthreads();
+        for (int i = t; i < RT * 16 * nt; i += GT) {  // (tile, row, token) sums over the slices in order
+            const int m = i / (16 * nt), r = (i / nt) % 16, tt = i % nt;
+            float sv = 0.0f;
 #pragma unroll
-            for (int m = 0; m < RT; ++m)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) red[((wave * RT + m) * 16 + 4 * lg + v) * MT + li] = acc[m][v];
-            __syncthreads();
-            for (int i = t; i < TW * 16 * nt; i += GT) {  // (tile, row, token) sums over the slices in order
-                const int k = i / (16 * nt), r = (i / nt) % 16, tt = i % nt;
-                const int kg = k / RT, m = k % RT;
-                float sv = 0.0f;
-#pragma unroll
-                for (int q = 0; q < KS; ++q) sv = sv + red[(((kg * KS + q) * RT + m) * 16 + r) * MT + tt];
-                ydn[(int64_t)plist[s0 + c0 + tt] * H + (u * TW + k) * 16 + r] = sv;
-            }
-            __syncthreads();
+            for (int q = 0; q < GW; ++q) sv = sv + red[((q * RT + m) * 16 + r) * MT + tt];
+            ydn[(int64_t)plist[s0 + c0 + tt] * H + (tile0 + m) * 16 + r] = sv;
         }
+        __syncthreads();
     }
 }
 
@@ -1096,6 +1217,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     const int gmax = std::min(E, P);
     const int gbig = std::min(gmax, n_mfma > P ? 0 : P / n_mfma);  // at most this many groups of >= n_mfma tokens
     const bool dot4 = n_mfma > 1, mfma = n_seqs >= n_mfma;
+    const int n_tiles = std::min(P, P / MT + gbig);  // at most this many token tiles
     if (mfma && (int64_t)P * nbj * Q8_BLK >= (int64_t)NO_TOKEN)
         return fail(FT_HIP_E_SHAPE, "%s: %d pairs x %d act blocks: the MFMA path's activation buffer must stay under 2 GiB",
                     nm, P, nbj);
@@ -1116,13 +1238,24 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         if ((rc = launch_status("moe_layer_grouped/gate_up"))) return rc;
     }
     if (mfma) {
-        const size_t lds_mg = (size_t)nb * 256 + sizeof(float) * (GW * 64 * MTP + MT * 64 + MT * 32) + 4 * MT * 10 +
-                              8 * MT + 4 * (size_t)MT * (nb * 10 + 1);
-        auto kern = H == 2816 ? (rec ? k_mfma_gu<11, true> : k_mfma_gu<11, false>)
-                              : (rec ? k_mfma_gu<16, true> : k_mfma_gu<16, false>);
-        const int grid = std::min(ctx->num_cus, nbj * gbig);  // persistent: one workgroup per CU
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(GT), lds_mg, s, (const uint8_t*)bank, eb, (const int32_t*)w.meta,
-                           (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, H, I, E, K, P, rgu);
+        auto gate_up = [&](auto kern, int nw, int kh) {
+            const size_t lds_mg = (size_t)nb / kh * ((MT * 8 + 2) * 4 + MT * 4) + (size_t)nw * nb / 8 * 128;
+            hipLaunchKernelGGL(kern, dim3(((nbj + nw - 1) / nw * n_tiles + 7) / 8 * 8), dim3(nw * 64), lds_mg, s,
+                               (const uint8_t*)bank, eb, (const int32_t*)w.meta, (const uint32_t*)w.ppos,
+                               (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, I, E, K, P, rgu);
+        };
+        // Two forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
+        // for all 128 of the Gemma shape), and small workgroups that hold half of the tokens' rows at a time
+        // (36 KB of LDS, 3 to a CU) spread them best over the CUs: 64 tokens 63 us against 73 for the other
+        // form, 127 tokens 64 against 73 (zipf-skewed 55 against 65). More tokens: the VALU bounds it, and 8
+        // waves share one staging of whole rows, two workgroups to a CU: 512 tokens 118-126 us against 137,
+        // 173 zipf-skewed tokens 67 against 70; at 10 pairs per expert 74 against 80 (zipf-skewed 67, 71).
+        if (H == 2816 && P < 9 * E)
+            gate_up(rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true> : k_mfma_gu_tok<11, 4, 3, 8, 2, false>, 4, 2);
+        else if (H == 2816)
+            gate_up(rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true> : k_mfma_gu_tok<11, 8, 4, 6, 1, false>, 8, 1);
+        else
+            gate_up(rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true> : k_mfma_gu_tok<16, 16, 4, 6, 1, false>, 16, 1);
         if ((rc = launch_status("moe_layer_grouped/gate_up_mfma"))) return rc;
         if (dbg_act) {  // the debug copy below reads q8a's pair rows
             hipLaunchKernelGGL(k_q8m_rows, dim3(64, (unsigned)gbig), dim3(256), 0, s,
@@ -1145,17 +1278,19 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         if ((rc = launch_status("moe_layer_grouped/down"))) return rc;
     }
     if (mfma) {
-        if (nbj <= 32) {  // one K slice: 8 waves x 2 tiles of 16 rows per workgroup
-            const size_t lds_md = (size_t)GW * 2 * nbj * 32 + sizeof(float) * GW * 2 * 16 * MT;
-            auto kern = rec ? k_mfma_down<1, 32, 2, 4, 2, true> : k_mfma_down<1, 32, 2, 4, 2, false>;
-            hipLaunchKernelGGL(kern, dim3(H / (16 * GW * 2), gbig), dim3(GT), lds_md, s, (const uint8_t*)bank, eb,
-                               gu_bytes, (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8m, P,
-                               w.ydn, H, I, E, n_mfma, rdn);
+        if (nbj <= 32) {
+            constexpr int NW = 4;
+            const size_t lds_md = (size_t)nbj * (576 + NW * 128);
+            auto kern = nbj <= 24 ? (rec ? k_mfma_down_tok<6, 2, NW, true> : k_mfma_down_tok<6, 2, NW, false>)
+                                  : (rec ? k_mfma_down_tok<8, 2, NW, true> : k_mfma_down_tok<8, 2, NW, false>);
+            hipLaunchKernelGGL(kern, dim3(((H / 64 + NW - 1) / NW * n_tiles + 7) / 8 * 8), dim3(NW * 64), lds_md, s,
+                               (const uint8_t*)bank, eb, gu_bytes, (const int32_t*)w.meta, (const uint32_t*)w.ppos,
+                               (const int32_t*)w.plist, (const uint8_t*)w.q8m, P, w.ydn, H, I, E, rdn);
         } else {  // long rows: DRT tiles per workgroup, 8 K slices of 56 (rows up to 448 blocks) or 64 blocks
             constexpr int DRT = 4;
             const size_t lds_md = std::max((size_t)DRT * nbj * 32, sizeof(float) * GW * DRT * 16 * MT);
-            auto kern = nbj <= 8 * 56 ? (rec ? k_mfma_down<GW, 56, DRT, 4, 2, true> : k_mfma_down<GW, 56, DRT, 4, 2, false>)
-                                      : (rec ? k_mfma_down<GW, 64, DRT, 4, 2, true> : k_mfma_down<GW, 64, DRT, 4, 2, false>);
+            auto kern = nbj <= 8 * 56 ? (rec ? k_mfma_down<56, DRT, 4, 2, true> : k_mfma_down<56, DRT, 4, 2, false>)
+                                      : (rec ? k_mfma_down<64, DRT, 4, 2, true> : k_mfma_down<64, DRT, 4, 2, false>);
             hipLaunchKernelGGL(kern, dim3(H / (16 * DRT), gbig), dim3(GT), lds_md, s, (const uint8_t*)bank, eb,
                                gu_bytes, (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8m, P,
                                w.ydn, H, I, E, n_mfma, rdn);

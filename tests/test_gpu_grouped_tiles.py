@@ -1,0 +1,69 @@
+"""GPU parity of the token-tile MFMA kernels of ft_hip_moe_layer_grouped at the
+edges of their tiles: experts with 0, 1, 15, 16, 17, 32 and 33 tokens (tiles
+of 16), act blocks that do not fill a workgroup's waves (inter 96, 416, 1024),
+both hidden sizes, and batches on both sides of the line between the two
+gate|up variants (9 pairs per expert). The dot4 kernels are the reference:
+they add the same block products in the same order, so gate|up sums and act
+blocks are the same bits; the down sums run in another order."""
+import numpy as np
+import pytest
+import torch
+
+import ft_hip
+import moe_synth
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("hidden,inter,counts", [
+    (2816, 96, [1, 15, 16, 17, 0, 2, 0, 3]),       # 54 pairs: under 9 per expert
+    (2816, 704, [1, 15, 16, 17, 32, 33, 0, 2]),    # 116 pairs: over
+    (2816, 1024, [33, 0, 0, 0, 0, 0, 0, 46]),      # 79 pairs: just under, two experts only
+    (2816, 416, [72, 0, 0, 0, 0, 0, 0, 0]),        # 72 pairs: on the line, one expert
+    (4096, 96, [17, 0, 1, 16, 0, 0, 0, 33]),
+])
+@pytest.mark.parametrize("norm", [False, True])
+def test_token_tiles_match_dot4(gemv, hidden, inter, counts, norm):
+    E, K, B = len(counts), 1, sum(counts)
+    src = torch.empty(E * moe_synth.expert_geometry(
+        moe_synth.Shape("t", hidden, inter, E, K, 1, 77), ft_hip.LAYOUT_Q4R)[2], dtype=torch.uint8, device=DEV)
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 77), ft_hip.LAYOUT_Q4R)
+    for e in range(E):
+        gemv.gen_q4_rows(1000 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(2000 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    rng = np.random.default_rng(hidden + inter + B)
+    who = rng.permutation(np.repeat(np.arange(E), counts))
+    X = rng.standard_normal((B, hidden)).astype(np.float32)
+    X[:, :E] = 0.0
+    X[np.arange(B), who] = 30.0  # the router picks the expert of this column
+    W = np.zeros((E, hidden), np.float32)
+    W[np.arange(E), np.arange(E)] = 1.0
+    x, w = torch.from_numpy(X).to(DEV), torch.from_numpy(W).to(DEV)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+    got = {}
+    try:
+        gemv.set_input_norm(norm)
+        for name, mfma_min in (("mfma", 1), ("dot4", 10**6)):
+            gemv.set_grouped_mfma_min(mfma_min)
+            out = torch.zeros_like(x)
+            ids = torch.zeros(B * K, dtype=torch.int32, device=DEV)
+            wts = torch.zeros(B * K, dtype=torch.float32, device=DEV)
+            gu = torch.zeros((B * K, 2 * inter), dtype=torch.float32, device=DEV)
+            act = torch.zeros((B * K, inter // 32, 40), dtype=torch.uint8, device=DEV)
+            gemv.moe_layer_grouped(x, out, B, hidden, inter, E, K, w, None, None, bank, ids, wts, ws, gu, act)
+            gemv.moe_layer_grouped(x, out, B, hidden, inter, E, K, w, None, None, bank, ids, wts, ws)
+            torch.cuda.synchronize()
+            assert np.array_equal(ids.cpu().numpy(), who)
+            got[name] = [t.cpu().numpy() for t in (gu, act, out)]
+    finally:
+        gemv.set_input_norm(0)
+        gemv.set_grouped_mfma_min(0)
+    assert np.array_equal(got["mfma"][0].view(np.uint32), got["dot4"][0].view(np.uint32))
+    assert np.array_equal(got["mfma"][1], got["dot4"][1])
+    # two orders of at most 32 block sums: 2 * 32 * 2^-24 = 4e-6 of the sum of
+    # their sizes, itself within 25 times the largest output
+    upd = got["dot4"][2] - X
+    assert np.max(np.abs(got["mfma"][2] - got["dot4"][2])) <= 1e-4 * np.max(np.abs(upd))
