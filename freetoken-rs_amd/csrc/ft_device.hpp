@@ -230,6 +230,30 @@ __device__ __forceinline__ uint64_t rank_key(float v, int i) {
     return ((uint64_t)mo << 32) | (0xFFFFFFFFu - (uint32_t)i);
 }
 
+// 4x4 transpose across the 16-lane rows of a wavefront: on entry lane row g
+// holds M[g][0..3] in (a0..a3), on exit T[g][j] = M[j][g]. Two 32-lane swaps
+// exchange the off-diagonal 2x2 blocks, two 16-lane swaps the off-diagonal
+// elements inside each block.
+__device__ __forceinline__ void quad_transpose(uint32_t& a0, uint32_t& a1, uint32_t& a2, uint32_t& a3) {
+    const auto s0 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
+    const auto s1 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
+    const auto s2 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
+    const auto s3 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
+    a0 = s2[0];
+    a1 = s2[1];
+    a2 = s3[0];
+    a3 = s3[1];
+}
+
+__device__ __forceinline__ void quad_transpose_f(float& a0, float& a1, float& a2, float& a3) {
+    uint32_t u0 = __float_as_uint(a0), u1 = __float_as_uint(a1), u2 = __float_as_uint(a2), u3 = __float_as_uint(a3);
+    quad_transpose(u0, u1, u2, u3);
+    a0 = __uint_as_float(u0);
+    a1 = __uint_as_float(u1);
+    a2 = __uint_as_float(u2);
+    a3 = __uint_as_float(u3);
+}
+
 // ---------------------------------------------------------------------------
 // GELU and the softmax exp with the bits of the libm calls ft-core makes
 // (f32::tanh, ft-model/src/lib.rs:436; f32::exp, :1495): restatements of

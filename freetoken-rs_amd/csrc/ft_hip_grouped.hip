@@ -545,21 +545,6 @@ __device__ __forceinline__ ActOp act_op_m(__amdgpu_buffer_rsrc_t r, uint32_t vq,
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// 4x4 transpose across the 16-lane rows of a wavefront: on entry lane row g
-// holds M[g][0..3] in (a0..a3), on exit T[g][j] = M[j][g]. Two 32-lane swaps
-// exchange the off-diagonal 2x2 blocks, two 16-lane swaps the off-diagonal
-// elements inside each block.
-__device__ __forceinline__ void quad_transpose(uint32_t& a0, uint32_t& a1, uint32_t& a2, uint32_t& a3) {
-    const auto s0 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
-    const auto s1 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
-    const auto s2 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
-    const auto s3 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
-    a0 = s2[0];
-    a1 = s2[1];
-    a2 = s3[0];
-    a3 = s3[1];
-}
-
 // A operand from qs word g of a row's block: low nibbles, then high nibbles.
 __device__ __forceinline__ long nib_op(uint32_t w) {
     return (long)(((uint64_t)((w >> 4) & 0x0F0F0F0Fu) << 32) | (w & 0x0F0F0F0Fu));
@@ -1179,7 +1164,12 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     const int64_t gu_bytes = 2LL * I * nb * 18;
     int rc;
     const float* inv = ctx->input_norm ? w.inv : nullptr;
-    if (n_experts * 16 >= hidden / 32) {  // logits, norm scale and q8(x) in one launch
+    const bool parts = ft::route_parts_fits(hidden, n_experts, top_k, n_seqs);
+    if (parts) {  // the whole routing; its group sums in ydn, which the down launch writes after their last reader
+        if ((rc = ft::launch_route_topk(stream, router_w, x, router_bias, expert_scale, ctx->input_norm, w.inv, w.q8x,
+                                        w.ydn, ids, wts, hidden, n_experts, top_k, n_seqs)))
+            return rc;
+    } else if (n_experts * 16 >= hidden / 32) {  // logits, norm scale and q8(x) in one launch
         if ((rc = ft::launch_route_prep(stream, router_w, x, router_bias, ctx->input_norm, w.inv, w.q8x, w.logits,
                                         hidden, n_experts, n_seqs)))
             return rc;
@@ -1193,8 +1183,8 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // to 4 rounds of 1024/E tokens), else its own launch: one workgroup
     // ranking 128 logits per token is LDS-bound (batch 16 of the Gemma
     // shape: 188.4 vs 172.6 us/token); at 8 experts it saves the launch
-    const bool topk_in = E <= 32 && n_seqs <= 4 * (1024 / E);
-    if (!topk_in && (rc = ft_hip_topk_router(ctx, stream, w.logits, expert_scale, ids, wts, n_experts, top_k, n_seqs)))
+    const bool topk_in = !parts && E <= 32 && n_seqs <= 4 * (1024 / E);
+    if (!topk_in && !parts && (rc = ft_hip_topk_router(ctx, stream, w.logits, expert_scale, ids, wts, n_experts, top_k, n_seqs)))
         return rc;
     // groups of >= n_mfma tokens take the MFMA tile kernels, the others the
     // dot4 kernels; rows longer than 32 blocks (I > 1024) only the former.

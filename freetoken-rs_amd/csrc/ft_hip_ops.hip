@@ -1197,6 +1197,109 @@ __global__ __launch_bounds__(256) void k_route_prep_m(const float* W, const floa
     }
 }
 
+// The head of a layer for many seqs, its dots on the matrix cores: workgroup
+// (x, y, g) forms the R-order's group g of the logits of 32 router rows and 32
+// seqs, a 16x16 tile per wave. v_mfma_f32_16x16x1 (four blocks) is one fma per
+// output, so 16 of them from zero are the chunk's fma chain of k_route_prep,
+// bit for bit, for four chunks at once (block b: chunk 4s + b); a lane holds
+// all four partials of its outputs and adds them to the group's sum in chunk
+// order. Out go the group sums, part [8][n_seqs][n_rows], and of the first
+// row tile the seqs' self-dots, ss [8][n_seqs] (norm; on the VALU beside), which
+// k_topk_parts sums over the groups. Each workgroup also quantizes its share of
+// the seqs' q8 blocks.
+//
+// What bounds it is bytes into a CU: a dot of f32 rows reads 4 bytes per fma and
+// operand row, so the groups go to different workgroups (90 KB each) rather
+// than 16 whole rows and seqs to one (360 KB: 16 us for any number of seqs),
+// and the rows come through LDS by contiguous reads: loaded where the lanes
+// need them, 16 rows a load, their stride (11,264 bytes) put them on 4 of the
+// L2's 16 channels (173 seqs 10.2 us against 7.4, 512 seqs 17.4 against 15.5;
+// k_route_prep_n and _m 22.5 and 30).
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <int C>
+__global__ __launch_bounds__(256) void k_route_parts(const float* __restrict__ W, const float* __restrict__ x, int norm,
+                                                    float* ss, uint8_t* q8, float* part, int dim, int n_rows,
+                                                    int n_seqs) {
+    constexpr int STEPS = (C + 3) / 4, RS = C * 16 + 4;  // chunks per group / 4; LDS row stride (words), 16 rows of a read on distinct banks
+    extern __shared__ __align__(16) float tile[];          // [32 router rows, then 32 seqs][RS]
+    __shared__ float P[2][4 * STEPS][16];                  // x.x chunk partials of the group
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63, b = l >> 4, r = l & 15;
+    const int g = blockIdx.z, ts = wave >> 1;
+    const int e0 = blockIdx.x * 32 + (wave & 1) * 16, t0 = blockIdx.y * 32 + ts * 16;
+    const bool dots = norm && blockIdx.x == 0 && (wave & 1) == 0;
+    constexpr int N = 64 * C * 4 / 256, HB = N / 2;  // float4 per thread, in two batches
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float4 v[HB];
+#pragma unroll
+        for (int i = 0; i < HB; ++i) {
+            const int f = (h * HB + i) * 256 + t, row = f / (C * 4), c4 = f - row * (C * 4);
+            const float* src = row < 32 ? W + (int64_t)(blockIdx.x * 32 + row) * dim
+                                        : x + (int64_t)min((int)blockIdx.y * 32 + row - 32, n_seqs - 1) * dim;
+            v[i] = reinterpret_cast<const float4*>(src + g * C * 16)[c4];
+        }
+#pragma unroll
+        for (int i = 0; i < HB; ++i) {
+            const int f = (h * HB + i) * 256 + t, row = f / (C * 4), c4 = f - row * (C * 4);
+            *reinterpret_cast<float4*>(tile + row * RS + c4 * 4) = v[i];
+        }
+    }
+    __syncthreads();
+    if (t0 < n_seqs) {  // uniform per wave
+        const float* wr = tile + ((wave & 1) * 16 + r) * RS;
+        const float* xr = tile + (32 + ts * 16 + r) * RS;
+        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int ck = min(4 * s + b, C - 1);  // past the group: its last chunk again, not added
+            v16f d = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            float p = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float4 a = *reinterpret_cast<const float4*>(wr + ck * 16 + 4 * k);
+                const float4 v = *reinterpret_cast<const float4*>(xr + ck * 16 + 4 * k);
+                d = __builtin_amdgcn_mfma_f32_16x16x1f32(a.x, v.x, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x1f32(a.y, v.y, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x1f32(a.z, v.z, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x1f32(a.w, v.w, d, 0, 0, 0);
+                p = fmaf(v.x, v.x, p);
+                p = fmaf(v.y, v.y, p);
+                p = fmaf(v.z, v.z, p);
+                p = fmaf(v.w, v.w, p);
+            }
+            if (dots) P[ts][4 * s + b][r] = p;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (4 * s + q < C) {  // uniform
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sum[v] = sum[v] + d[4 * q + v];
+                }
+        }
+        if (t0 + r < n_seqs)  // rows 4b..4b+3 of seq r
+            *reinterpret_cast<float4*>(part + ((int64_t)g * n_seqs + t0 + r) * n_rows + e0 + 4 * b) =
+                make_float4(sum[0], sum[1], sum[2], sum[3]);
+    }
+    if (norm && blockIdx.x == 0) {  // uniform
+        __syncthreads();
+        const int s = blockIdx.y * 32 + t;
+        if (t < 32 && s < n_seqs) {
+            float v = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4 * STEPS; ++c)
+                if (c < C) v = v + P[t >> 4][c][r];
+            ss[(int64_t)g * n_seqs + s] = v;
+        }
+    }
+    // q8 blocks [sh*Q, sh*Q + Q) of the 32 seqs, sh this workgroup's share
+    const int nb = dim >> 5, ns = gridDim.x * 8, sh = blockIdx.x * 8 + g, Q = (nb + ns - 1) / ns;
+    for (int i = t; i < 32 * Q * 4; i += 256) {  // whole quads: 4 consecutive lanes per block
+        const int q = i / (Q * 4), rem = i - q * Q * 4, bk = sh * Q + (rem >> 2), s = blockIdx.y * 32 + q;
+        if (s < n_seqs && bk < nb)
+            quantize_block_quad(x + (int64_t)s * dim + 32 * bk, rem & 3,
+                                reinterpret_cast<uint32_t*>(q8 + ((int64_t)s * nb + bk) * Q8_BLK));
+    }
+}
+
 // Scale of the input RMS norm per seq: inv[s] = 1 / sqrt(ss / dim + 1e-6),
 // ss = x_s.x_s in the R-order, each op rounded once. Grid n_seqs.
 __global__ __launch_bounds__(256) void k_rms_inv(const float* x, float* inv, int dim) {
@@ -1268,6 +1371,44 @@ __global__ __launch_bounds__(256) void k_topk_router(const float* logits, const 
         __syncthreads();
     }
     __shared__ float exv[32];
+    const float w = topk_softmax(selv, seli, k, escale, exv);
+    if (t < k) {
+        ids[(int64_t)s * k + t] = seli[t];
+        wts[(int64_t)s * k + t] = w;
+    }
+}
+
+// k_topk_router for up to 256 experts from k_route_parts' group sums: the
+// logit of a thread's expert is their sum in group order, times the norm's
+// scale, plus the bias (k_route_prep's arithmetic). Stores inv.
+__global__ __launch_bounds__(256) void k_topk_parts(const float* part, const float* ss, const float* bias, int norm,
+                                                    float* inv, const float* escale, int32_t* ids, float* wts, int E,
+                                                    int k, int dim) {
+    __shared__ float sv[256], selv[32], exv[32];
+    __shared__ int seli[32];
+    __shared__ uint64_t key[256];
+    const int s = blockIdx.x, t = threadIdx.x, n = gridDim.x, e = min(t, E - 1);
+    float pv[8], sq[8];
+#pragma unroll
+    for (int g = 0; g < 8; ++g) pv[g] = part[((int64_t)g * n + s) * E + e];
+#pragma unroll
+    for (int g = 0; g < 8; ++g) sq[g] = norm ? ss[(int64_t)g * n + s] : 0.0f;
+    const float bv = bias ? bias[e] : 0.0f;
+    float lg = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) lg = lg + pv[g];
+    if (norm) {
+        float q = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) q = q + sq[g];
+        const float ir = 1.0f / sqrtf(q / (float)dim + 1e-6f);  // correctly rounded (HIP default)
+        lg = lg * ir;
+        if (t == 0) inv[s] = ir;
+    }
+    if (bias) lg = lg + bv;
+    if (t < E) sv[t] = lg;
+    __syncthreads();
+    topk_rank_select(sv, E, k, key, selv, seli);
     const float w = topk_softmax(selv, seli, k, escale, exv);
     if (t < k) {
         ids[(int64_t)s * k + t] = seli[t];
@@ -1771,6 +1912,26 @@ int launch_route_prep(void* stream, const float* w, const float* x, const float*
     hipLaunchKernelGGL(k_route_prep, dim3((unsigned)n_rows, (unsigned)n_seqs), dim3(256), (size_t)(dim / 16) * 8,
                        S(stream), w, x, bias, norm, inv, (uint8_t*)q8, y, (int)dim, (int)n_rows);
     return launch_status("route_prep");
+}
+
+bool route_parts_fits(int64_t dim, int64_t n_rows, int64_t top_k, int64_t n_seqs) {
+    // up to 64 seqs launch_route_prep's VALU forms are as fast (64 seqs, both launches: 13.7 us against 14.0; 16
+    // seqs 11.0 against 12.8); past them the group sums are (173: 28.4 against 14.4, 512: 36.6 against 23.5)
+    return n_seqs > 64 && (dim == 2816 || dim == 4096) && n_rows % 32 == 0 && n_rows <= 256 &&
+           8 * (n_rows + 1) <= top_k * dim;
+}
+
+int launch_route_topk(void* stream, const float* w, const float* x, const float* bias, const float* escale, int norm,
+                      float* inv, void* q8, float* part, int32_t* ids, float* wts, int64_t dim, int64_t n_rows,
+                      int64_t top_k, int64_t n_seqs) {
+    float* ss = part + 8 * n_seqs * n_rows;
+    auto kern = dim == 2816 ? k_route_parts<22> : k_route_parts<32>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_rows / 32), (unsigned)((n_seqs + 31) / 32), 8), dim3(256),
+                       64 * (size_t)(dim / 8 + 4) * sizeof(float), S(stream), w, x, norm, ss, (uint8_t*)q8, part, (int)dim, (int)n_rows, (int)n_seqs);
+    if (int rc = launch_status("route_parts")) return rc;
+    hipLaunchKernelGGL(k_topk_parts, dim3((unsigned)n_seqs), dim3(256), 0, S(stream), (const float*)part,
+                       (const float*)ss, bias, norm, inv, escale, ids, wts, (int)n_rows, (int)top_k, (int)dim);
+    return launch_status("topk_parts");
 }
 
 int launch_rms_inv(void* stream, const float* x, float* inv, int64_t dim, int64_t n_seqs) {

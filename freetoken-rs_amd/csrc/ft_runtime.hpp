@@ -56,6 +56,15 @@ int launch_router_logits(void* stream, const float* w, const float* x, const flo
 // needs n_rows * 16 >= dim / 32.
 int launch_route_prep(void* stream, const float* w, const float* x, const float* bias, int norm, float* inv,
                       void* q8, float* y, int64_t dim, int64_t n_rows, int64_t n_seqs);
+// Routing of many seqs in two launches on the matrix cores (the same bits as
+// launch_route_prep and ft_hip_topk_router): q8(x), the norm's scale and the
+// top-k; part: scratch of 8 * n_seqs * (n_rows + 1) floats. For shapes
+// route_parts_fits takes (it also says that top_k * dim floats per seq are
+// scratch enough).
+bool route_parts_fits(int64_t dim, int64_t n_rows, int64_t top_k, int64_t n_seqs);
+int launch_route_topk(void* stream, const float* w, const float* x, const float* bias, const float* escale, int norm,
+                      float* inv, void* q8, float* part, int32_t* ids, float* wts, int64_t dim, int64_t n_rows,
+                      int64_t top_k, int64_t n_seqs);
 // Resolves the no-alloc scratch array's device address for ctx->device
 // (current) into ctx->noalloc_scratch (ft_hip_ops.hip, beside the array).
 int scratch_setup(ft_hip_ctx* ctx);

@@ -19,7 +19,7 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("hidden,inter,counts", [
     (2816, 96, [1, 15, 16, 17, 0, 2, 0, 3]),       # 54 pairs: under 9 per expert
     (2816, 704, [1, 15, 16, 17, 32, 33, 0, 2]),    # 116 pairs: over
-    (2816, 1024, [33, 0, 0, 0, 0, 0, 0, 46]),      # 79 pairs: just under, two experts only
+    (2816, 1024, [33, 0, 0, 0, 0, 0, 0, 38]),      # 71 pairs: just under, two experts only
     (2816, 416, [72, 0, 0, 0, 0, 0, 0, 0]),        # 72 pairs: on the line, one expert
     (4096, 96, [17, 0, 1, 16, 0, 0, 0, 33]),
 ])
@@ -67,3 +67,47 @@ def test_token_tiles_match_dot4(gemv, hidden, inter, counts, norm):
     # their sizes, itself within 25 times the largest output
     upd = got["dot4"][2] - X
     assert np.max(np.abs(got["mfma"][2] - got["dot4"][2])) <= 1e-4 * np.max(np.abs(upd))
+
+
+@pytest.mark.parametrize("hidden,E,K,B", [(2816, 128, 8, 65), (2816, 128, 8, 97), (2816, 32, 1, 161), (4096, 256, 4, 96)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_routing_of_many_seqs_matches_few(gemv, hidden, E, K, B, norm):
+    """Past 64 seqs the routing goes through group sums on the matrix cores: the
+    same ids and weights, bit for bit, as calls of up to 64 seqs each, at batches
+    that do not fill the last tile of 32 seqs; and the same layer output."""
+    inter = 32
+    rng = np.random.default_rng(hidden + E + B)
+    x = torch.from_numpy(rng.standard_normal((B, hidden)).astype(np.float32)).to(DEV)
+    w = torch.from_numpy((rng.standard_normal((E, hidden)) * 0.02).astype(np.float32)).to(DEV)
+    bias = torch.from_numpy(rng.standard_normal(E).astype(np.float32)).to(DEV)
+    scale = torch.from_numpy(rng.uniform(0.5, 2.0, E).astype(np.float32)).to(DEV)
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 78), ft_hip.LAYOUT_Q4R)
+    src = torch.empty(E * eb, dtype=torch.uint8, device=DEV)
+    for e in range(E):
+        gemv.gen_q4_rows(3000 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(4000 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+
+    def layer(part):
+        n = len(part)
+        out = torch.zeros_like(part)
+        ids = torch.zeros(n * K, dtype=torch.int32, device=DEV)
+        wts = torch.zeros(n * K, dtype=torch.float32, device=DEV)
+        gemv.moe_layer_grouped(part, out, n, hidden, inter, E, K, w, bias, scale, bank, ids, wts, ws)
+        torch.cuda.synchronize()
+        return out.cpu().numpy(), ids.cpu().numpy().reshape(n, K), wts.cpu().numpy().reshape(n, K)
+
+    try:
+        gemv.set_input_norm(norm)
+        gemv.set_grouped_mfma_min(1)
+        out, ids, wts = layer(x)
+        for t0 in range(0, B, 48):
+            o, i, v = layer(x[t0:t0 + 48].contiguous())
+            assert np.array_equal(i, ids[t0:t0 + 48])
+            assert np.array_equal(v.view(np.uint32), wts[t0:t0 + 48].view(np.uint32))
+            assert np.array_equal(o.view(np.uint32), out[t0:t0 + 48].view(np.uint32))
+    finally:
+        gemv.set_input_norm(0)
+        gemv.set_grouped_mfma_min(0)
