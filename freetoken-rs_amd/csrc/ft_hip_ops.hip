@@ -7,6 +7,7 @@
 #include "ft_runtime.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace ft;
 
@@ -58,13 +59,9 @@ __device__ __forceinline__ void load_block(const uint8_t* wr, int b, int qs_off,
         d4 = h2f(reinterpret_cast<const uint16_t*>(wr)[b]);
         q = *reinterpret_cast<const uint4*>(wr + qs_off + 16 * b);
     } else {
-        // 18-byte blocks are only 2-byte aligned: nine u16 loads.
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(wr + 18 * b);
-        d4 = h2f(p[0]);
-        q.x = (uint32_t)p[1] | ((uint32_t)p[2] << 16);
-        q.y = (uint32_t)p[3] | ((uint32_t)p[4] << 16);
-        q.z = (uint32_t)p[5] | ((uint32_t)p[6] << 16);
-        q.w = (uint32_t)p[7] | ((uint32_t)p[8] << 16);
+        // 18-byte blocks are only 2-byte aligned; global loads take any alignment, so the 16 bytes are one load
+        d4 = h2f(*reinterpret_cast<const uint16_t*>(wr + 18 * b));
+        __builtin_memcpy(&q, wr + 18 * b + 2, 16);
     }
 }
 
@@ -173,10 +170,36 @@ __device__ __forceinline__ float topk_softmax(const float* selv, const int* seli
     return w;
 }
 
+// Four blocks of a row, b, b+step, ...: their loads issued together (past the
+// row's end its last block again, not used).
+template <int LAYOUT>
+struct Blocks4 {
+    float d4[4];
+    uint4 q[4];
+    __device__ __forceinline__ void load(const uint8_t* wr, int b, int step, int nb, int qs_off) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load_block<LAYOUT>(wr, min(b + step * u, nb - 1), qs_off, d4[u], q[u]);
+    }
+    // the blocks below nb onto acc, in order
+    template <bool REC>
+    __device__ __forceinline__ float dots(float acc, int b, int step, int nb, const int* lds, int32_t* rec) const {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int bb = b + step * u;
+            const int* xb = lds + min(bb, nb - 1) * 10;
+            const float d8 = __int_as_float(xb[0]);
+            const int diff = block_dot(q[u], xb + 2, xb[1]);
+            if constexpr (REC) if (rec && bb < nb) rec[bb] = diff;
+            acc = bb < nb ? fmaf((float)diff, d4[u] * d8, acc) : acc;
+        }
+        return acc;
+    }
+};
+
 // One row's share of a lane: lane `sub` of the row's LPR takes blocks sub,
 // sub+LPR, ..., an fma chain in block order (four blocks' loads issued
-// together: long rows are otherwise one load latency per block). The caller
-// sums the LPR lanes by xor 1, 2, 4 (, 8).
+// together, the last one to four as well: a row is otherwise one load latency
+// per block). The caller sums the LPR lanes by xor 1, 2, 4 (, 8).
 template <int LAYOUT, int LPR = 8, bool REC = false>
 __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int nb, const int* lds,
                                                int32_t* rec = nullptr) {
@@ -197,15 +220,54 @@ __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int n
             acc = fmaf((float)diff, d4[u] * d8, acc);
         }
     }
-    for (; b < nb; b += LPR) {
-        float d4;
-        uint4 q;
-        load_block<LAYOUT>(wr, b, qs_off, d4, q);
-        const int* xb = lds + b * 10;
-        const float d8 = __int_as_float(xb[0]);
-        const int diff = block_dot(q, xb + 2, xb[1]);
-        if constexpr (REC) if (rec) rec[b] = diff;
-        acc = fmaf((float)diff, d4 * d8, acc);
+    if constexpr (LPR <= 8) {
+        if (b < nb) {
+            Blocks4<LAYOUT> k;
+            k.load(wr, b, LPR, nb, qs_off);
+            acc = k.template dots<REC>(acc, b, LPR, nb, lds, rec);
+        }
+    } else {  // long rows: the tail is a small part, and its code costs the loop above (large-expert stack 1 %)
+        for (; b < nb; b += LPR) {
+            float d4;
+            uint4 q;
+            load_block<LAYOUT>(wr, b, qs_off, d4, q);
+            const int* xb = lds + b * 10;
+            const float d8 = __int_as_float(xb[0]);
+            const int diff = block_dot(q, xb + 2, xb[1]);
+            if constexpr (REC) if (rec) rec[b] = diff;
+            acc = fmaf((float)diff, d4 * d8, acc);
+        }
+    }
+    return acc;
+}
+
+// gemv_row_part's four-lane chains (lane s: blocks s, s+4, ...) with two lanes on
+// each: lane u of chain s loads and dots blocks s + 4*(2*i + u), six rounds'
+// loads at once, and hands its dots and scale products to the other, and both
+// add them in block order: the bits of gemv_row_part<LAYOUT, 4>. The caller sums
+// the chains by xor 2, 4.
+template <int LAYOUT, bool REC>
+__device__ __forceinline__ float gemv_row_chain(const uint8_t* wr, int s, int u, int nb, const int* lds,
+                                                int32_t* rec) {
+    constexpr int R = 6, WU = 2;
+    const int qs_off = (nb * 2 + 15) / 16 * 16;
+    float acc = 0.0f;
+    for (int i0 = 0; 4 * WU * i0 < nb; i0 += R) {  // uniform
+        float d4[R];
+        uint4 q[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            load_block<LAYOUT>(wr, min(s + 4 * (WU * (i0 + r) + u), nb - 1), qs_off, d4[r], q[r]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int b0 = s + 4 * WU * (i0 + r), b = b0 + 4 * u;
+            const int* xb = lds + min(b, nb - 1) * 10;
+            const int diff = block_dot(q[r], xb + 2, xb[1]);
+            const float f = (float)diff, sc = d4[r] * __int_as_float(xb[0]);
+            if constexpr (REC) if (rec && b < nb) rec[b] = diff;
+            acc = b0 < nb ? fmaf(dpp_f<0xA0>(f), dpp_f<0xA0>(sc), acc) : acc;
+            acc = b0 + 4 < nb ? fmaf(dpp_f<0xF5>(f), dpp_f<0xF5>(sc), acc) : acc;
+        }
     }
     return acc;
 }
@@ -403,7 +465,8 @@ __device__ __forceinline__ void record_sums(const GemvArgs& a, int e, int inter,
 // row (gemv_row_part), and writes q8 block j of the pair's activation with
 // k_gelu_mul_q8's arithmetic. LPR 8 gives k_gemv_q4_grouped's sums (and so
 // the bits of the two launches); LPR 4 sums each row in 4 lane chains.
-// Grid (I/32, n_pairs).
+// Grid (I/32, n_pairs). WU: lanes per chain (LPR 4, gemv_row_chain), WU times
+// the threads: the same bits.
 //
 // TOPK: the routing of the pair's seq (top-div of the E <= 256 logits and
 // their softmax, the arithmetic of k_topk_router) is computed by every
@@ -421,8 +484,8 @@ __device__ __forceinline__ void record_sums(const GemvArgs& a, int e, int inter,
 // a.dots[pair][row][block], the scaled gate and up sums it hands to GELU to
 // a.sums[pair][row], and (HEAD) the seq's first workgroup the q8 row of x it
 // computed to a.x8rec[seq]; null pointers are skipped.
-template <int LAYOUT, bool TOPK, int LPR = 8, bool HEAD = false, bool REC = false>
-__global__ __launch_bounds__(64 * LPR, 24 / LPR) void k_gemv_gu_act(GemvArgs a, int inter, uint8_t* q8a,
+template <int LAYOUT, bool TOPK, int LPR = 8, bool HEAD = false, bool REC = false, int WU = 1>
+__global__ __launch_bounds__(64 * LPR * WU, WU == 1 ? 24 / LPR : 1) void k_gemv_gu_act(GemvArgs a, int inter, uint8_t* q8a,
                                                                   const float* in_scale, int div, const float* logits,
                                                                   const float* escale, int32_t* ids, float* wts,
                                                                   int E, HeadArgs h) {
@@ -460,14 +523,23 @@ __global__ __launch_bounds__(64 * LPR, 24 / LPR) void k_gemv_gu_act(GemvArgs a, 
     }
     const uint8_t* eb = a.base + (uint64_t)slot * a.expert_bytes + a.bank_off;
     const int nb = a.k >> 5;
-    // waves 0..LPR/2-1: gate rows, the others up rows, 64/LPR rows per wave
+    // the first half of the waves: gate rows, the others up rows, 64/(LPR*WU) rows per wave
+    constexpr int L = LPR * WU;  // lanes per row
     const int lane = t & 63, wave = t >> 6;
-    const bool up = wave >= LPR / 2;
-    const int rl = (wave - (up ? LPR / 2 : 0)) * (64 / LPR) + lane / LPR, sub = lane % LPR;
+    const bool up = wave >= L / 2;
+    const int rl = (wave - (up ? L / 2 : 0)) * (64 / L) + lane / L, sub = lane % L;
     const int row = (up ? inter : 0) + (int)blockIdx.x * 32 + rl;
     int32_t* rec = REC && a.dots ? a.dots + ((int64_t)e * 2 * inter + row) * nb : nullptr;
-    float acc = gemv_row_part<LAYOUT, LPR, REC>(eb + (int64_t)row * row_bytes_of(LAYOUT, a.k), sub, nb, lds, rec);
-    acc = sum_row_lanes<LPR>(acc);
+    const uint8_t* wr = eb + (int64_t)row * row_bytes_of(LAYOUT, a.k);
+    float acc;
+    if constexpr (WU == 1) {
+        acc = sum_row_lanes<LPR>(gemv_row_part<LAYOUT, LPR, REC>(wr, sub, nb, lds, rec));
+    } else {
+        static_assert(LPR == 4 && WU == 2, "gemv_row_chain");
+        acc = gemv_row_chain<LAYOUT, REC>(wr, sub / WU, sub % WU, nb, lds, rec);
+        acc += __shfl_xor(acc, WU);
+        acc += __shfl_xor(acc, 2 * WU);
+    }
     if (sub == 0) gs[(up ? 32 : 0) + rl] = acc;
     __syncthreads();
     if (threadIdx.x < 64) {  // both half-waves compute block j; the first stores it
@@ -492,8 +564,10 @@ __global__ __launch_bounds__(64 * LPR, 24 / LPR) void k_gemv_gu_act(GemvArgs a, 
 // + ...) for them, pairs in order. LPR lanes per row: 8 is
 // k_gemv_q4_grouped's arithmetic; 16 (long rows) sums each row's blocks in
 // 16 lane chains instead, twice the workgroups. Grid (ceil(H/R), n_seqs).
+// SHORT (rows of up to 4*LPR blocks): a lane's blocks are all loaded before the
+// activation rows are staged, one latency for both.
 // REC (test record): every int32 block dot also goes to a.dots[pair][row][block].
-template <int LAYOUT, int LPR, bool REC = false>
+template <int LAYOUT, int LPR, bool SHORT, bool REC>
 __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const float* wts, const float* x, float* out,
                                                            int k) {
     extern __shared__ int lds[];
@@ -501,19 +575,23 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     __shared__ float ys[NE];
     const int s = blockIdx.y, R = NE / k;
     const int nb = a.k >> 5;
-    // up to 40 loads per thread in one batch: the k rows (36 words per thread
-    // for two rows of 448 blocks) arrive in one load latency
-    stage_words<40>(reinterpret_cast<const int*>(a.q8 + (int64_t)s * k * a.q8_stride_blocks * Q8_BLK), k * nb * 10,
-                    lds);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int re = wave * (64 / LPR) + lane / LPR, sub = lane % LPR;  // row entry: pair kk, local row rl
     const int kk = re / R, rl = re - kk * R;
     const int row = (int)blockIdx.x * R + rl;
+    const bool live = row < a.n_rows;
+    const uint8_t* wr = entry_base(a, s * k + kk) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k);
+    Blocks4<LAYOUT> w4;
+    if constexpr (SHORT) w4.load(wr, sub, LPR, nb, (nb * 2 + 15) / 16 * 16);  // the row's share, with the q8 rows
+    // up to 40 loads per thread in one batch: the k rows (36 words per thread
+    // for two rows of 448 blocks) arrive in one load latency
+    stage_words<40>(reinterpret_cast<const int*>(a.q8 + (int64_t)s * k * a.q8_stride_blocks * Q8_BLK), k * nb * 10,
+                    lds);
     float acc = 0.0f;
-    if (row < a.n_rows) {
+    if (live) {
         int32_t* rec = REC && a.dots ? a.dots + ((int64_t)(s * k + kk) * a.n_rows + row) * nb : nullptr;
-        acc = gemv_row_part<LAYOUT, LPR, REC>(entry_base(a, s * k + kk) + (int64_t)row * row_bytes_of(LAYOUT, a.k),
-                                              sub, nb, lds + kk * nb * 10, rec);
+        if constexpr (SHORT) acc = sub < nb ? w4.template dots<REC>(0.0f, sub, LPR, nb, lds + kk * nb * 10, rec) : 0.0f;
+        else acc = gemv_row_part<LAYOUT, LPR, REC>(wr, sub, nb, lds + kk * nb * 10, rec);
     }
     acc = sum_row_lanes<LPR>(acc);
     if (sub == 0) ys[re] = acc;
@@ -1625,19 +1703,21 @@ static void launch_gu_long(int bpl, dim3 grid, size_t lds, hipStream_t st, const
                                             wts, E, h);
 }
 
-// The gate|up launch with the activation, k_gemv_gu_act<LAYOUT, TOPK,
-// GU_LANES, HEAD> or its record instantiation.
+// The gate|up launch with the activation, k_gemv_gu_act. q4r rows: two lanes
+// on each of a row's four chains (Gemma shape, gate|up launch: 12.1 us against
+// 13.0 for 1 token, 34.6 against 38.9 for 8; four lanes 12.3 and 59); q4_0
+// rows one (8 tokens 39.9 us against 42.4 with two).
 template <bool TOPK, bool HEAD>
 static void launch_gu_act(int layout, bool rec, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a, int inter,
                           uint8_t* q8a, const float* in_scale, int div, const float* logits, const float* escale,
                           int32_t* ids, float* wts, int E, const HeadArgs& h) {
-    auto kern = layout == FT_LAYOUT_Q4R
-                    ? (rec ? k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, true>
-                           : k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, false>)
+    const bool q4r = layout == FT_LAYOUT_Q4R;
+    auto kern = q4r ? (rec ? k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, true, 2>
+                           : k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, false, 2>)
                     : (rec ? k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, true>
                            : k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, false>);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * GU_LANES), lds, st, a, inter, q8a, in_scale, div, logits, escale, ids,
-                       wts, E, h);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * GU_LANES * (q4r ? 2 : 1)), lds, st, a, inter, q8a, in_scale, div, logits,
+                       escale, ids, wts, E, h);
 }
 
 template <int LPR, bool REC, int XIN = 0, bool ACT = false>
@@ -2320,15 +2400,16 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
         const bool l16 = down_lanes(inter, top_k) == 16;
         const int R = (int)((l16 ? 16 : 32) / top_k);
         const dim3 g_dn((unsigned)((hidden + R - 1) / R), (unsigned)n_seqs);
-        auto kern = layout == FT_LAYOUT_Q4R
-                        ? (l16 ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, 16, true>
-                                         : k_gemv_down_combine<FT_LAYOUT_Q4R, 16, false>)
-                               : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, 8, true>
-                                         : k_gemv_down_combine<FT_LAYOUT_Q4R, 8, false>))
-                        : (l16 ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, 16, true>
-                                         : k_gemv_down_combine<FT_LAYOUT_Q4_0, 16, false>)
-                               : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, 8, true>
-                                         : k_gemv_down_combine<FT_LAYOUT_Q4_0, 8, false>));
+        const bool q4r = layout == FT_LAYOUT_Q4R;
+        auto pick = [&](auto lpr, auto sh) {
+            constexpr int L = decltype(lpr)::value;
+            constexpr bool SH = decltype(sh)::value;
+            return q4r ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, L, SH, true> : k_gemv_down_combine<FT_LAYOUT_Q4R, L, SH, false>)
+                       : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, L, SH, true> : k_gemv_down_combine<FT_LAYOUT_Q4_0, L, SH, false>);
+        };
+        auto kern = l16 ? pick(std::integral_constant<int, 16>{}, std::false_type{})
+                    : inter / 32 <= 32 ? pick(std::integral_constant<int, 8>{}, std::true_type{})
+                                       : pick(std::integral_constant<int, 8>{}, std::false_type{});
         hipLaunchKernelGGL(kern, g_dn, dim3(256), l_dn, st, a, (const float*)wts, x, x_out, (int)top_k);
         return launch_status("moe_layer/down_combine");
     }
