@@ -64,6 +64,8 @@
 #include "ft_device.hpp"
 #include "ft_runtime.hpp"
 
+#include <algorithm>
+
 using namespace ft;
 
 namespace {
@@ -1463,12 +1465,10 @@ __device__ __forceinline__ void src_block(const uint8_t* row, int layout, int nb
         d = reinterpret_cast<const uint16_t*>(row)[b];
         q = *reinterpret_cast<const uint4*>(row + qs_off + 16 * b);
     } else {
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(row + 18 * b);
-        d = p[0];
-        q.x = (uint32_t)p[1] | ((uint32_t)p[2] << 16);
-        q.y = (uint32_t)p[3] | ((uint32_t)p[4] << 16);
-        q.z = (uint32_t)p[5] | ((uint32_t)p[6] << 16);
-        q.w = (uint32_t)p[7] | ((uint32_t)p[8] << 16);
+        d = *reinterpret_cast<const uint16_t*>(row + 18 * b);
+        typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+        const u32x4_u v = *reinterpret_cast<const u32x4_u*>(row + 18 * b + 2);  // global loads take any alignment
+        q = make_uint4(v.x, v.y, v.z, v.w);
     }
 }
 
@@ -1477,47 +1477,70 @@ __host__ __device__ __forceinline__ int64_t rowb(int layout, int k) {
     return layout == FT_LAYOUT_Q4R ? (int64_t)((nb * 2 + 15) / 16 * 16) + (int64_t)nb * 16 : (int64_t)nb * 18;
 }
 
-// one thread per (expert, gate|up tile jb, block b, lane r)
-__global__ __launch_bounds__(256) void k_pack_gu(const uint8_t* src, int layout, int64_t src_eb, uint8_t* dst,
-                                                 int64_t dst_eb, int H, int I, int64_t n_experts) {
-    const int nb = H >> 5, nbj = I >> 5;
-    const int64_t per_e = (int64_t)nbj * nb * 64;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n_experts * per_e) return;
-    const int64_t e = g / per_e;
-    int64_t rem = g % per_e;
-    const int jb = (int)(rem / (nb * 64));
-    rem %= nb * 64;
-    const int b = (int)(rem / 64), r = (int)(rem % 64);
-    const int row = r < 32 ? jb * 32 + r : I + jb * 32 + (r - 32);
-    uint16_t d;
-    uint4 q;
-    src_block(src + e * src_eb + row * rowb(layout, H), layout, nb, b, d, q);
-    uint8_t* T = dst + e * dst_eb + (int64_t)jb * nb * 1152;
-    *reinterpret_cast<uint16_t*>(T + b * 128 + r * 2) = d;
-    *reinterpret_cast<uint4*>(T + nb * 128 + b * 1024 + r * 16) = q;
-}
-
-// one thread per (expert, down tile jt, block b, row r)
-__global__ __launch_bounds__(256) void k_pack_dn(const uint8_t* src, int layout, int64_t src_eb, uint8_t* dst,
-                                                 int64_t dst_eb, int H, int I, int64_t n_experts) {
-    const int nbj = I >> 5, nt = H / DN_ROWS;
-    const int64_t per_e = (int64_t)nt * nbj * DN_ROWS;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n_experts * per_e) return;
-    const int64_t e = g / per_e;
-    int64_t rem = g % per_e;
-    const int jt = (int)(rem / (nbj * DN_ROWS));
-    rem %= nbj * DN_ROWS;
-    const int b = (int)(rem / DN_ROWS), r = (int)(rem % DN_ROWS);
-    const int64_t src_gu = 2LL * I * rowb(layout, H);
-    const int64_t dst_gu = 2LL * I * (H / 32) * 18;
-    uint16_t d;
-    uint4 q;
-    src_block(src + e * src_eb + src_gu + (int64_t)(jt * DN_ROWS + r) * rowb(layout, I), layout, nbj, b, d, q);
-    uint8_t* T = dst + e * dst_eb + dst_gu + (int64_t)jt * nbj * 288;
-    *reinterpret_cast<uint16_t*>(T + b * 32 + r * 2) = d;
-    *reinterpret_cast<uint4*>(T + nbj * 32 + b * 256 + r * 16) = q;
+// Rows to fused tiles through LDS: a workgroup takes 64 rows by PK_B blocks of
+// one expert (DOWN: of its down rows, four 16-row tiles; else gate|up tile
+// blockIdx.y). Read along the rows (PK_B blocks contiguous), written along the
+// tile's blocks; both copies are memory-bound, and one block per thread straight
+// from a row to its tile read a 128-byte line per 18 bytes (a layer's 128
+// experts of the Gemma shape, read and written: 244 us).
+constexpr int PK_B = 16;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <bool DOWN, int LAYOUT>
+__global__ __launch_bounds__(256) void k_pack(const uint8_t* src, int64_t src_eb, uint8_t* dst,
+                                              int64_t dst_eb, int H, int I, int64_t n_experts) {
+    constexpr int N = 64 * PK_B / 256, QS = 64 * 16 + 16;  // items per thread; LDS bytes per block, padded
+    __shared__ __align__(16) uint8_t qs[PK_B * QS];
+    __shared__ uint16_t ds[PK_B][64];
+    const int k = DOWN ? I : H, nb = k >> 5, rows = DOWN ? H : 2 * I, t = threadIdx.x;
+    const int b0 = blockIdx.x * PK_B, r0 = blockIdx.y * 64;
+    const int64_t src0 = DOWN ? 2LL * I * rowb(LAYOUT, H) : 0, dst0 = DOWN ? 2LL * I * (H / 32) * 18 : 0;
+    for (int64_t e = blockIdx.z; e < n_experts; e += gridDim.z) {
+        const uint8_t* S = src + e * src_eb + src0;
+        uint8_t* D = dst + e * dst_eb + dst0;
+        uint16_t d[N] = {};
+        u32x4 q[N] = {};
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int rr = (i * 256 + t) / PK_B, b = b0 + t % PK_B;
+            const int row = DOWN ? r0 + rr : (rr < 32 ? blockIdx.y * 32 + rr : I + blockIdx.y * 32 + rr - 32);
+            if (b < nb && row < rows) {
+                uint16_t dv;
+                uint4 v;
+                src_block(S + row * rowb(LAYOUT, k), LAYOUT, nb, b, dv, v);
+                d[i] = dv;
+                q[i] = u32x4{v.x, v.y, v.z, v.w};
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int rr = (i * 256 + t) / PK_B, b = t % PK_B;
+            ds[b][rr] = d[i];
+            *reinterpret_cast<u32x4*>(qs + b * QS + rr * 16) = q[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int it = i * 256 + t;
+            if constexpr (DOWN) {  // tile, block, row of 16
+                const int tt = it / (PK_B * 16), b = it / 16 % PK_B, r = it % 16, row = r0 + tt * 16 + r;
+                uint8_t* T = D + (int64_t)(row / 16) * nb * 288;
+                if (b0 + b < nb && row < rows) {
+                    *reinterpret_cast<uint16_t*>(T + (b0 + b) * 32 + r * 2) = ds[b][tt * 16 + r];
+                    *reinterpret_cast<uint4*>(T + nb * 32 + (b0 + b) * 256 + r * 16) =
+                        *reinterpret_cast<const uint4*>(qs + b * QS + (tt * 16 + r) * 16);
+                }
+            } else {
+                const int b = it / 64, r = it % 64;
+                uint8_t* T = D + (int64_t)blockIdx.y * nb * 1152;
+                if (b0 + b < nb) {
+                    *reinterpret_cast<uint16_t*>(T + (b0 + b) * 128 + r * 2) = ds[b][r];
+                    *reinterpret_cast<uint4*>(T + nb * 128 + (int64_t)(b0 + b) * 1024 + r * 16) =
+                        *reinterpret_cast<const uint4*>(qs + b * QS + r * 16);
+                }
+            }
+        }
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(256) void k_pack_router(const float* src, float* dst, int64_t n_layers, int E, int H) {
@@ -1736,13 +1759,17 @@ extern "C" int ft_hip_pack_experts_fused(ft_hip_ctx* ctx, void* stream, const vo
     if (n_experts == 0) return FT_HIP_OK;
     const int64_t eb = ft_hip_fused_expert_bytes(hidden, inter);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const int64_t n1 = n_experts * (inter / 32) * (hidden / 32) * 64;
-    hipLaunchKernelGGL(k_pack_gu, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, s, (const uint8_t*)src, src_layout,
-                       (int64_t)src_expert_bytes, (uint8_t*)dst, eb, (int)hidden, (int)inter, n_experts);
+    const unsigned ez = (unsigned)std::min<int64_t>(n_experts, 65535);
+    const bool q4r = src_layout == FT_LAYOUT_Q4R;
+    hipLaunchKernelGGL((q4r ? k_pack<false, FT_LAYOUT_Q4R> : k_pack<false, FT_LAYOUT_Q4_0>),
+                       dim3((unsigned)((hidden / 32 + PK_B - 1) / PK_B), (unsigned)(inter / 32), ez), dim3(256), 0, s,
+                       (const uint8_t*)src, (int64_t)src_expert_bytes, (uint8_t*)dst, eb, (int)hidden, (int)inter,
+                       n_experts);
     if (int rc = launch_status(nm)) return rc;
-    const int64_t n2 = n_experts * (hidden / DN_ROWS) * (inter / 32) * DN_ROWS;
-    hipLaunchKernelGGL(k_pack_dn, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, s, (const uint8_t*)src, src_layout,
-                       (int64_t)src_expert_bytes, (uint8_t*)dst, eb, (int)hidden, (int)inter, n_experts);
+    hipLaunchKernelGGL((q4r ? k_pack<true, FT_LAYOUT_Q4R> : k_pack<true, FT_LAYOUT_Q4_0>),
+                       dim3((unsigned)((inter / 32 + PK_B - 1) / PK_B), (unsigned)((hidden + 63) / 64), ez), dim3(256),
+                       0, s, (const uint8_t*)src, (int64_t)src_expert_bytes, (uint8_t*)dst, eb, (int)hidden, (int)inter,
+                       n_experts);
     return launch_status(nm);
 }
 
