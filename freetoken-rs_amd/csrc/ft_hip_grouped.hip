@@ -1188,12 +1188,14 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         return rc;
     // groups of >= n_mfma tokens take the MFMA tile kernels, the others the
     // dot4 kernels; rows longer than 32 blocks (I > 1024) only the former.
-    // Automatic (0): every group on one family, MFMA from 4 pairs per expert
-    // on (measured on the Gemma shape: dot4 faster at 1 pair per expert,
-    // 168.9 vs 217.5 us/token at batch 16; MFMA at 4, 73.5 vs 76.7 at batch
-    // 64, and above; one family's launches beat a split of both)
+    // Automatic (0): every group on one family, MFMA from 2/3 of a pair per
+    // expert on (its grouping, gate|up and down launches against dot4's two, on
+    // the Gemma shape with uniform / zipf-skewed routing: 8 tokens 58.7 / 42.0
+    // us against 51.0 / 45.4, 11 tokens 60.8 / 42.9 against 60.7 / 60.1, 16
+    // tokens 71.3 / 45.7 against 76.9 / 79.2, 63 tokens 101 / 67 against 146 /
+    // 246: dot4's cost grows with an expert's tokens)
     int n_mfma = ctx->grouped_mfma_min;
-    if (n_mfma <= 0) n_mfma = (int64_t)P >= 4 * n_experts ? 1 : std::numeric_limits<int>::max();
+    if (n_mfma <= 0) n_mfma = 3LL * P >= 2 * n_experts ? 1 : std::numeric_limits<int>::max();
     if (nbj > 32) n_mfma = 1;
     // every expert on the dot4 kernels, routing already in ids: the dot4
     // workgroups find their expert's pairs themselves (no grouping launch)

@@ -379,8 +379,8 @@ int ft_hip_moe_stack_grouped(ft_hip_ctx* ctx, void* stream, const float* x_in, f
  * v_mfma_i32_16x16x32_i8, one q4_0 block per instruction), the others the
  * v_dot4 kernels; results agree to f32 summation order (q8 quants, int32
  * block dots, routing and GELU q8 are the same). 0 (the default) = automatic:
- * every expert on the MFMA kernels when the batch has at least 4 (token,
- * expert) pairs per expert (n_seqs * top_k >= 4 * n_experts), else every
+ * every expert on the MFMA kernels when the batch has at least 2/3 of a (token,
+ * expert) pair per expert (3 * n_seqs * top_k >= 2 * n_experts), else every
  * expert on the dot4 kernels; 1 = MFMA
  * for every expert. Rows longer than 1024 weights (inter > 1024) always take
  * the MFMA kernels. No reference counterpart (the reference runs one GEMV
