@@ -42,7 +42,7 @@ struct GroupWs {
     uint8_t* q8x;       // [B][H/32][40]
     int32_t* meta;      // [0] active experts; [1..] gexp[E], gstart[E], gcount[E]; [1+3E] MFMA groups
     int32_t* plist;     // [P] pairs grouped by expert
-    int32_t* ppos;      // [P] scratch
+    int32_t* ppos;      // [P] token tiles of the MFMA groups (tile_entry)
     uint8_t* q8a;       // [P][I/32][40]
     uint8_t* q8m;       // the MFMA groups' act quants by group position q: [I/32][4][P] (qs words g, g+4), then [I/32][P] (d, qsum)
     float* ydn;         // [P][H]
@@ -172,10 +172,15 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
     auto pid = [&](int p) { return TOPK ? sid[p] : ids[p]; };
     for (int e = t; e < E; e += 1024) cnt[e] = 0;
     __syncthreads();
-    for (int p = t; p < P; p += 1024) {
-        const int e = min(max(pid(p), 0), E - 1);
-        ppos[p] = atomicAdd(&cnt[e], 1);
+    // a thread's pairs, their experts and places in registers (P <= MAX_PAIRS)
+    int ex[MAX_PAIRS / 1024], at[MAX_PAIRS / 1024];
+#pragma unroll
+    for (int i = 0; i < MAX_PAIRS / 1024; ++i) {
+        const int p = i * 1024 + t;
+        ex[i] = p < P ? min(max(pid(p), 0), E - 1) : 0;
     }
+#pragma unroll
+    for (int i = 0; i < MAX_PAIRS / 1024; ++i) at[i] = i * 1024 + t < P ? atomicAdd(&cnt[ex[i]], 1) : 0;
     __syncthreads();
     // inclusive prefix sums of counts and of "active" / "big" flags (E <=
     // 1024): within each wavefront by shuffles, then each thread adds the
@@ -226,11 +231,10 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
         meta[1 + 3 * E] = big[1023];
     }
     __syncthreads();
-    for (int p = t; p < P; p += 1024) {
-        const int e = min(max(pid(p), 0), E - 1);
-        plist[scan[e] - cnt[e] + ppos[p]] = p;
-    }
-    __syncthreads();  // ppos is read: it becomes the tile list (every tile holds a pair, so P entries suffice)
+#pragma unroll
+    for (int i = 0; i < MAX_PAIRS / 1024; ++i)
+        if (i * 1024 + t < P) plist[scan[ex[i]] - cnt[ex[i]] + at[i]] = i * 1024 + t;
+    // the tile list (every tile holds a pair, so P entries suffice)
     for (int k = 0; k < my_tiles; ++k) ppos[vt - my_tiles + k] = (int32_t)tile_entry(n_tiles, big[t] - 1, k * MT);
     if (t == 0 && n_tiles == 0) ppos[0] = 0;
 }
