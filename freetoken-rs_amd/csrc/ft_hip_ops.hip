@@ -286,21 +286,29 @@ __device__ __forceinline__ float sum_row_lanes(float acc) {
 // rows of one entry: 8 lanes per row, lane s takes blocks s, s+8, ...; the
 // activation sits in LDS. REC: every block's int32 dot is also stored to
 // a.dots[e][row][block] (test record). Grid: (ceil(n_rows/32), n_entries).
-template <int LAYOUT, bool REC>
+// SHORT (rows of up to 32 blocks): a lane's blocks are loaded before the
+// activation row is staged, one latency for both.
+template <int LAYOUT, bool REC, bool SHORT = false>
 __global__ __launch_bounds__(256) void k_gemv_q4_grouped(GemvArgs a) {
     extern __shared__ int lds[];
     const int e = blockIdx.y;
-    stage_q8(a, e, lds);
     const int nb = a.k >> 5;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = (blockIdx.x * 4 + wave) * 8 + (lane >> 3);
     const int sub = lane & 7;
+    const bool live = row < a.n_rows;
+    const uint8_t* wr = entry_base(a, e) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k);
+    Blocks4<LAYOUT> w4;
+    if constexpr (SHORT) w4.load(wr, sub, 8, nb, (nb * 2 + 15) / 16 * 16);
+    stage_q8(a, e, lds);
     float acc = 0.0f;
-    if (row < a.n_rows)
-        acc = gemv_row_part<LAYOUT, 8, REC>(entry_base(a, e) + (int64_t)row * row_bytes_of(LAYOUT, a.k), sub, nb,
-                                            lds, REC ? a.dots + ((int64_t)e * a.n_rows + row) * nb : nullptr);
+    if (live) {
+        int32_t* rec = REC ? a.dots + ((int64_t)e * a.n_rows + row) * nb : nullptr;
+        if constexpr (SHORT) acc = w4.template dots<REC>(0.0f, sub, 8, nb, lds, rec);
+        else acc = gemv_row_part<LAYOUT, 8, REC>(wr, sub, nb, lds, rec);
+    }
     acc = sum_row_lanes(acc);
-    if (row < a.n_rows && sub == 0) a.y[(int64_t)e * a.y_stride + row] = acc;
+    if (live && sub == 0) a.y[(int64_t)e * a.y_stride + row] = acc;
 }
 
 // Short-launch GEMV for q4r matrices whose k_gemv_q4_grouped grid would
@@ -1809,12 +1817,15 @@ static int gemv_common(ft_hip_ctx* ctx, void* stream, GemvArgs& a, int64_t n_ent
         if (lpr == 16) launch_short<16>(rec, nbl, g2, lds, S(stream), a);
         else if (lpr == 32) launch_short<32>(rec, nbl, g2, lds, S(stream), a);
         else launch_short<64>(rec, nbl, g2, lds, S(stream), a);
-    } else if (layout == FT_LAYOUT_Q4R) {
-        hipLaunchKernelGGL((rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4R, true> : k_gemv_q4_grouped<FT_LAYOUT_Q4R, false>),
-                           grid, dim3(256), lds, S(stream), a);
     } else {
-        hipLaunchKernelGGL((rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4_0, true> : k_gemv_q4_grouped<FT_LAYOUT_Q4_0, false>),
-                           grid, dim3(256), lds, S(stream), a);
+        const bool q4r = layout == FT_LAYOUT_Q4R;
+        auto pick = [&](auto sh) {
+            constexpr bool SH = decltype(sh)::value;
+            return q4r ? (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4R, true, SH> : k_gemv_q4_grouped<FT_LAYOUT_Q4R, false, SH>)
+                       : (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4_0, true, SH> : k_gemv_q4_grouped<FT_LAYOUT_Q4_0, false, SH>);
+        };
+        hipLaunchKernelGGL(nb <= 32 ? pick(std::true_type{}) : pick(std::false_type{}), grid, dim3(256), lds, S(stream),
+                           a);
     }
     return launch_status(name);
 }
