@@ -269,8 +269,10 @@ __device__ __forceinline__ int scan_pairs(const int32_t* ids, int P, int e, int*
 // Gate|up tile j of active expert g for all of its tokens, then GELU*up and
 // the q8 of act block j per token. BPW = H/32/8 blocks per wave. in_scale
 // (input RMS norm, or null): a token's gate|up sums are first multiplied by
-// in_scale[token]. SCAN: the grid's y is the expert, whose pairs the
-// workgroup finds in ids[0..P) (scan_pairs) instead of the group list.
+// in_scale[token]. SCAN: the grid's y is the expert, or a pair
+// if there are fewer of those (empty workgroups: 2,046 of 2,816 at 5 tokens of
+// the Gemma shape, now 110 of 880), and the workgroup finds its expert's pairs
+// in ids[0..P) (scan_pairs) instead of the group list.
 template <int BPW, bool REC, bool SCAN>
 __global__ __launch_bounds__(GT, 2) void k_grouped_gu(const uint8_t* bank, int64_t expert_bytes, const int32_t* meta,
                                                       const int32_t* plist, const uint8_t* q8x, uint8_t* q8a,
@@ -284,9 +286,11 @@ __global__ __launch_bounds__(GT, 2) void k_grouped_gu(const uint8_t* bank, int64
     int e, n;
     const int32_t* lst;
     if constexpr (SCAN) {
-        e = blockIdx.y;
+        // fewer pairs than experts: the grid's y is a pair, and the expert's first pair takes the expert
+        const bool by_pair = P < E;
+        e = by_pair ? min(max(ids[blockIdx.y], 0), E - 1) : (int)blockIdx.y;
         n = scan_pairs(ids, P, e, slst, wcnt);
-        if (n == 0) return;
+        if (n == 0 || (by_pair && slst[0] != (int)blockIdx.y)) return;
         lst = slst;
     } else {
         const int g = blockIdx.y + meta[1 + 3 * E];  // after the MFMA kernels' groups
@@ -424,9 +428,11 @@ __global__ __launch_bounds__(GT, 1) void k_grouped_down(const uint8_t* bank, int
     int e, n;
     const int32_t* lst;
     if constexpr (SCAN) {
-        e = blockIdx.y;
+        // fewer pairs than experts: the grid's y is a pair, and the expert's first pair takes the expert
+        const bool by_pair = P < E;
+        e = by_pair ? min(max(ids[blockIdx.y], 0), E - 1) : (int)blockIdx.y;
         n = scan_pairs(ids, P, e, slst, wcnt);
-        if (n == 0) return;
+        if (n == 0 || (by_pair && slst[0] != (int)blockIdx.y)) return;
         lst = slst;
     } else {
         const int g = blockIdx.y + meta[1 + 3 * E];  // after the MFMA kernels' groups
@@ -1228,7 +1234,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
                                       : (rec ? k_grouped_gu<16, true, true> : k_grouped_gu<16, false, true>))
                          : (H == 2816 ? (rec ? k_grouped_gu<11, true, false> : k_grouped_gu<11, false, false>)
                                       : (rec ? k_grouped_gu<16, true, false> : k_grouped_gu<16, false, false>));
-        hipLaunchKernelGGL(kern, dim3(nbj, scan ? E : gmax), dim3(GT), lds_gu, s, (const uint8_t*)bank, eb,
+        hipLaunchKernelGGL(kern, dim3(nbj, gmax), dim3(GT), lds_gu, s, (const uint8_t*)bank, eb,
                            (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8a, dbg_gu, inv, H,
                            I, E, K, n_mfma, rgu, (const int32_t*)ids, P);
         if ((rc = launch_status("moe_layer_grouped/gate_up"))) return rc;
@@ -1268,7 +1274,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
                                       : (rec ? k_grouped_down<8, true, true> : k_grouped_down<8, false, true>))
                          : (nbj <= 24 ? (rec ? k_grouped_down<6, true, false> : k_grouped_down<6, false, false>)
                                       : (rec ? k_grouped_down<8, true, false> : k_grouped_down<8, false, false>));
-        hipLaunchKernelGGL(kern, dim3(H / DU, scan ? E : gmax), dim3(GT), lds_dn, s, (const uint8_t*)bank, eb, gu_bytes,
+        hipLaunchKernelGGL(kern, dim3(H / DU, gmax), dim3(GT), lds_dn, s, (const uint8_t*)bank, eb, gu_bytes,
                            (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8a, w.ydn, H, I, E,
                            n_mfma, rdn, (const int32_t*)ids, P);
         if ((rc = launch_status("moe_layer_grouped/down"))) return rc;
