@@ -588,9 +588,10 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     const int kk = re / R, rl = re - kk * R;
     const int row = (int)blockIdx.x * R + rl;
     const bool live = row < a.n_rows;
-    const uint8_t* wr = entry_base(a, s * k + kk) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k);
+    // the row's address depends on a slot load: a long row's is formed after the staging, whose loads it would hold up
+    auto wrow = [&] { return entry_base(a, s * k + kk) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k); };
     Blocks4<LAYOUT> w4;
-    if constexpr (SHORT) w4.load(wr, sub, LPR, nb, (nb * 2 + 15) / 16 * 16);  // the row's share, with the q8 rows
+    if constexpr (SHORT) w4.load(wrow(), sub, LPR, nb, (nb * 2 + 15) / 16 * 16);  // the row's share, with the q8 rows
     // up to 40 loads per thread in one batch: the k rows (36 words per thread
     // for two rows of 448 blocks) arrive in one load latency
     stage_words<40>(reinterpret_cast<const int*>(a.q8 + (int64_t)s * k * a.q8_stride_blocks * Q8_BLK), k * nb * 10,
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     if (live) {
         int32_t* rec = REC && a.dots ? a.dots + ((int64_t)(s * k + kk) * a.n_rows + row) * nb : nullptr;
         if constexpr (SHORT) acc = sub < nb ? w4.template dots<REC>(0.0f, sub, LPR, nb, lds + kk * nb * 10, rec) : 0.0f;
-        else acc = gemv_row_part<LAYOUT, LPR, REC>(wr, sub, nb, lds + kk * nb * 10, rec);
+        else acc = gemv_row_part<LAYOUT, LPR, REC>(wrow(), sub, nb, lds + kk * nb * 10, rec);
     }
     acc = sum_row_lanes<LPR>(acc);
     if (sub == 0) ys[re] = acc;
