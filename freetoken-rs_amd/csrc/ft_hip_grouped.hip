@@ -997,7 +997,7 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
             if constexpr (NBB == 4) {
 #pragma unroll
                 for (int m = 0; m < RT; ++m) {
-                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, 0);
+                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, 2);
                     aw[buf][0][m] = v.x;
                     aw[buf][1][m] = v.y;
                     aw[buf][2][m] = v.z;
