@@ -815,22 +815,25 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
 // from q8m as they lie (each block's words of a lane group contiguous over the
 // group's tokens) and are staged in LDS once for the workgroup's waves; the
 // rows stream through registers four blocks (NBUF - 1 batches) ahead. Per
-// (row, token) acc = fma(float(D_b), d4_b * d8_b, acc) in block order. Four
+// (row, token) acc = fma(float(D_b), d4_b * d8_b, acc) in block order, or with
+// LANES k_grouped_down's sums, bit for bit: four chains of blocks 4k, 4k + 1, ...,
+// products rounded before they are added, the chains as (0 + 1) + (2 + 3). Its
+// 48 registers more leave three waves a SIMD, and a layer of 11 to 63 tokens of the
+// Gemma shape takes 0.8 to 1.8 us longer (uniform routing 16 tokens 85.8 us against
+// 84.9, 63 tokens 120.3 against 118.5). Four
 // waves of about 94 registers per workgroup, several to a CU, so that one's
 // staging runs under another's dots (8 waves 64 us against 57 at 512 tokens;
 // two batches ahead instead of one 58.5). Before, one workgroup walked all of
 // an expert's tokens, rereading the weights for each 16: 512 tokens of the
 // Gemma shape 104 us, 173 zipf-skewed 93, 64 tokens 47; now 57, 31 and 33
 // (143 MB of weights, 4.4 TB/s).
-template <int NKB, int NBUF, int NW, bool REC>
-__global__ __launch_bounds__(NW * 64, 4) void k_mfma_down_tok(const uint8_t* __restrict__ bank, int64_t expert_bytes,
-                                                               int64_t gu_bytes, const int32_t* __restrict__ meta,
-                                                               const uint32_t* __restrict__ tiles,
-                                                               const int32_t* __restrict__ plist,
-                                                               const uint8_t* __restrict__ q8m, int P, float* ydn, int H,
-                                                               int I, int E, int32_t* rec) {
+template <int NKB, int NW, bool LANES, bool REC>
+__global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
+    const uint8_t* __restrict__ bank, int64_t expert_bytes, int64_t gu_bytes, const int32_t* __restrict__ meta,
+    const uint32_t* __restrict__ tiles, const int32_t* __restrict__ plist, const uint8_t* __restrict__ q8m, int P,
+    float* ydn, int H, int I, int E, int32_t* rec) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int NTH = NW * 64;
+    constexpr int NTH = NW * 64, NC = LANES ? 4 : 1, NBUF = 2;
     const int nbj = I >> 5, dn_tile = nbj * 288, RG = H / 64, JG = (RG + NW - 1) / NW;
     const int n_units = (int)(tiles[0] >> 18) * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
     const int unit = ((int)blockIdx.x & 7) * per + ur;  // as k_mfma_gu_tok's
@@ -884,11 +887,9 @@ __global__ __launch_bounds__(NW * 64, 4) void k_mfma_down_tok(const uint8_t* __r
         if (lane * 16 < nbj * 32) *reinterpret_cast<u32x4*>(scl + m * nbj * 32 + lane * 16) = ss[m];
     __syncthreads();
     if (rw0 >= RG) return;
-    float acc[4][4];
+    float acc[NC][4][4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[m][v] = 0.0f;
+    for (int i = 0; i < NC * 16; ++i) acc[i >> 4][i >> 2 & 3][i & 3] = 0.0f;
     const int p = plist[s0 + c0 + min(li, nt - 1)];
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
@@ -928,9 +929,11 @@ __global__ __launch_bounds__(NW * 64, 4) void k_mfma_down_tok(const uint8_t* __r
                             for (int v = 0; v < 4; ++v)
                                 rec[((int64_t)p * H + rg * 64 + m * 16 + 4 * lg + v) * nbj + blk] = d[m][v] >> 4;
                     }
+                    float(&a)[4] = acc[b % NC][m];
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[m][v] = fmaf((float)d[m][v], sp[m][v], acc[m][v]);
-                    asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
+                    for (int v = 0; v < 4; ++v)
+                        a[v] = LANES ? a[v] + (float)d[m][v] * sp[m][v] : fmaf((float)d[m][v], sp[m][v], a[v]);
+                    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
                 }
             }
             __builtin_amdgcn_sched_barrier(0);  // one block's MFMA results live at a time
@@ -938,9 +941,16 @@ __global__ __launch_bounds__(NW * 64, 4) void k_mfma_down_tok(const uint8_t* __r
     }
     if (li < nt) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int m = 0; m < 4; ++m) {
+            float y[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                y[v] = acc[0][m][v];
+                if constexpr (LANES) y[v] = (y[v] + acc[1][m][v]) + (acc[2][m][v] + acc[3][m][v]);
+            }
             *reinterpret_cast<float4*>(ydn + (int64_t)p * H + rg * 64 + m * 16 + 4 * lg) =
-                make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
+                make_float4(y[0], y[1], y[2], y[3]);
+        }
     }
 }
 
@@ -1207,6 +1217,11 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     int n_mfma = ctx->grouped_mfma_min;
     if (n_mfma <= 0) n_mfma = 3LL * P >= 2 * n_experts ? 1 : std::numeric_limits<int>::max();
     if (nbj > 32) n_mfma = 1;
+    // Automatic, below 4 pairs per expert: the down sums in the dot4 kernels' order, so that where the line above
+    // lies in this range shows in no output bit (another order of 22 block sums moves q8 quants of the layers that
+    // follow: 3e-4 of the state after four layers). From there on, and where the caller splits the experts, one chain
+    // in block order, the faster form.
+    const bool lanes = ctx->grouped_mfma_min <= 0 && P < 4LL * n_experts;
     // every expert on the dot4 kernels, routing already in ids: the dot4
     // workgroups find their expert's pairs themselves (no grouping launch)
     const bool scan = !topk_in && n_mfma > P && P <= SCAN_MAX;
@@ -1283,8 +1298,12 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         if (nbj <= 32) {
             constexpr int NW = 4;
             const size_t lds_md = (size_t)nbj * (576 + NW * 128);
-            auto kern = nbj <= 24 ? (rec ? k_mfma_down_tok<6, 2, NW, true> : k_mfma_down_tok<6, 2, NW, false>)
-                                  : (rec ? k_mfma_down_tok<8, 2, NW, true> : k_mfma_down_tok<8, 2, NW, false>);
+            auto pick = [&](auto ln) {
+                constexpr bool LN = decltype(ln)::value;
+                return nbj <= 24 ? (rec ? k_mfma_down_tok<6, NW, LN, true> : k_mfma_down_tok<6, NW, LN, false>)
+                                 : (rec ? k_mfma_down_tok<8, NW, LN, true> : k_mfma_down_tok<8, NW, LN, false>);
+            };
+            auto kern = lanes ? pick(std::true_type{}) : pick(std::false_type{});
             hipLaunchKernelGGL(kern, dim3(((H / 64 + NW - 1) / NW * n_tiles + 7) / 8 * 8), dim3(NW * 64), lds_md, s,
                                (const uint8_t*)bank, eb, gu_bytes, (const int32_t*)w.meta, (const uint32_t*)w.ppos,
                                (const int32_t*)w.plist, (const uint8_t*)w.q8m, P, w.ydn, H, I, E, rdn);

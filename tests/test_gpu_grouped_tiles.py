@@ -4,7 +4,9 @@ of 16), act blocks that do not fill a workgroup's waves (inter 96, 416, 1024),
 both hidden sizes, and batches on both sides of the line between the two
 gate|up variants (9 pairs per expert). The dot4 kernels are the reference:
 they add the same block products in the same order, so gate|up sums and act
-blocks are the same bits; the down sums run in another order."""
+blocks are the same bits; the down sums run in another order where the caller
+asks for the MFMA kernels, and in the same one where the automatic choice
+takes them below 4 pairs per expert."""
 import numpy as np
 import pytest
 import torch
@@ -108,6 +110,49 @@ def test_routing_of_many_seqs_matches_few(gemv, hidden, E, K, B, norm):
             assert np.array_equal(i, ids[t0:t0 + 48])
             assert np.array_equal(v.view(np.uint32), wts[t0:t0 + 48].view(np.uint32))
             assert np.array_equal(o.view(np.uint32), out[t0:t0 + 48].view(np.uint32))
+    finally:
+        gemv.set_input_norm(0)
+        gemv.set_grouped_mfma_min(0)
+
+
+@pytest.mark.parametrize("hidden,inter,E,K,B", [
+    (2816, 704, 128, 8, 11),   # 88 pairs: the first batch on the MFMA kernels
+    (2816, 704, 128, 8, 20),
+    (2816, 704, 128, 8, 63),   # 504 pairs: the last one under 4 per expert
+    (2816, 800, 9, 2, 17),     # 25 act blocks; experts of over 16 tokens
+    (4096, 1024, 9, 3, 11),    # 32 act blocks
+    (4096, 32, 40, 1, 159),    # one act block, three of the four chains empty
+    (2816, 96, 3, 1, 11),
+])
+@pytest.mark.parametrize("norm", [False, True])
+def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, inter, E, K, B, norm):
+    """Below 4 pairs per expert the automatic choice between the dot4 and the
+    MFMA kernels shows in no bit of the output: equal routing and uneven alike."""
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 79), ft_hip.LAYOUT_Q4R)
+    src = torch.empty(E * eb, dtype=torch.uint8, device=DEV)
+    for e in range(E):
+        gemv.gen_q4_rows(5000 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(6000 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    rng = np.random.default_rng(hidden + inter + B)
+    x = torch.from_numpy(rng.standard_normal((B, hidden)).astype(np.float32)).to(DEV)
+    w = torch.from_numpy((rng.standard_normal((E, hidden)) * 0.02).astype(np.float32)).to(DEV)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+    try:
+        gemv.set_input_norm(norm)
+        for bias in (None, torch.linspace(4, -4, E, device=DEV)):
+            got = []
+            for mfma_min in (0, 10**6):
+                gemv.set_grouped_mfma_min(mfma_min)
+                out = torch.zeros_like(x)
+                ids = torch.zeros(B * K, dtype=torch.int32, device=DEV)
+                wts = torch.zeros(B * K, dtype=torch.float32, device=DEV)
+                gemv.moe_layer_grouped(x, out, B, hidden, inter, E, K, w, bias, None, bank, ids, wts, ws)
+                torch.cuda.synchronize()
+                got.append([t.cpu().numpy().view(np.uint32) for t in (out, ids, wts)])
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
     finally:
         gemv.set_input_norm(0)
         gemv.set_grouped_mfma_min(0)
