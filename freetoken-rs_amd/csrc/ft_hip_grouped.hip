@@ -594,6 +594,83 @@ __device__ __forceinline__ void scales4(const uint16_t* p, float (&sc)[4]) {
     sc[3] = h2f((uint16_t)(s2.y >> 16));
 }
 
+// A token tile found without the grouping launch (SCAN, up to TILE_SCAN pairs
+// and 256 experts): the experts' tiles in expert order, a tile's pairs
+// ascending. Every wave does it by itself, in LDS of its own (its LDS
+// operations complete in order), so there is no barrier. For the down launch the
+// workgroup of each tile's first act blocks leaves a record: expert | tokens << 16, then the
+// 16 slots' pairs of 16 bits.
+constexpr int TILE_SCAN = 512;
+constexpr int TREC = 10;  // words per record (of GroupWs::q8a, a pair's act block, which a SCAN layer does not write)
+struct TileScan {
+    static constexpr int R = TILE_SCAN / 64;
+    int ex[R];       // the experts of pairs r * 64 + lane
+    int cn[4];       // the pair counts of experts 4 * lane ..
+    int first, end;  // the tiles of these experts
+    int e, c0, n;
+
+    __device__ __forceinline__ static void order() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // Counts the pairs per expert (cnt: 256 words of the wave); the number of tiles.
+    __device__ __forceinline__ int count(const int32_t* ids, int P, int E, int* cnt) {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int r = 0; r < R; ++r) ex[r] = r * 64 + lane < P ? min(max(ids[r * 64 + lane], 0), E - 1) : -1;
+        *reinterpret_cast<int4*>(cnt + 4 * lane) = make_int4(0, 0, 0, 0);
+        order();
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (ex[r] >= 0) atomicAdd(&cnt[ex[r]], 1);
+        order();
+        const int4 c = *reinterpret_cast<const int4*>(cnt + 4 * lane);
+        cn[0] = c.x;
+        cn[1] = c.y;
+        cn[2] = c.z;
+        cn[3] = c.w;
+        int tiles = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tiles += (cn[k] + MT - 1) / MT;
+        end = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int u = __shfl_up(end, d);
+            if (lane >= d) end += u;
+        }
+        first = end - tiles;
+        return __builtin_amdgcn_readlane(end, 63);
+    }
+    // Tile k's expert, first token and the expert's token count, and its pairs into tok[MT].
+    __device__ __forceinline__ void find(int k, int P, int* tok) {
+        const int lane = threadIdx.x & 63;
+        int at = first, ei = 0, ci = 0, ni = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int m = (cn[q] + MT - 1) / MT;
+            const bool hit = k >= at && k < at + m;
+            ei = hit ? 4 * lane + q : ei;
+            ci = hit ? (k - at) * MT : ci;
+            ni = hit ? cn[q] : ni;
+            at += m;
+        }
+        const int src = __ffsll((unsigned long long)__ballot(k >= first && k < end)) - 1;
+        e = __builtin_amdgcn_readlane(ei, src);
+        c0 = __builtin_amdgcn_readlane(ci, src);
+        n = __builtin_amdgcn_readlane(ni, src);
+        int base = -c0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r * 64 >= P) break;  // uniform
+            const uint64_t bal = __ballot(ex[r] == e);
+            const int i = base + __popcll(bal & ((1ull << lane) - 1));
+            if (ex[r] == e && i >= 0 && i < MT) tok[i] = r * 64 + lane;
+            base += __popcll(bal);
+        }
+        order();
+    }
+};
+
 // Gate|up of the MFMA groups by token tiles: workgroup (x, y) takes act blocks
 // x*NW .. x*NW + NW-1 (one wave each: the 64 rows of tile j) for tile y of the
 // token tiles that k_group_pairs lists (up to 16*TT tokens of one expert).
@@ -618,14 +695,12 @@ __device__ __forceinline__ void scales4(const uint16_t* p, float (&sc)[4]) {
 // matrix cores, 24 for operands and 10 for the GELU epilogue); for few the
 // weights (64 tokens: 285 MB in 63 us, 4.5 TB/s). Blocks are consumed one at a
 // time (sched_barrier), else the registers of a whole slice's dots spill.
-template <int BPW, int NW, int WPE, int D, int KH, bool REC>
-__global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __restrict__ bank, int64_t expert_bytes,
-                                                         const int32_t* __restrict__ meta,
-                                                         const uint32_t* __restrict__ tiles,
-                                                         const int32_t* __restrict__ plist,
-                                                         const uint8_t* __restrict__ q8x, uint8_t* q8m, float* dbg_gu,
-                                                         const float* __restrict__ in_scale, int I, int E, int K, int P,
-                                                         int32_t* rec) {
+template <int BPW, int NW, int WPE, int D, int KH, bool REC, bool SCAN>
+__global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
+    const uint8_t* __restrict__ bank, int64_t expert_bytes, const int32_t* __restrict__ meta, uint32_t* tiles,
+    const int32_t* __restrict__ plist, const uint8_t* __restrict__ q8x, uint8_t* q8m, float* dbg_gu,
+    const float* __restrict__ in_scale, int I, int E, int K, int P, int32_t* rec, const int32_t* __restrict__ ids,
+    uint32_t* trec) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int NB = 8 * BPW, TM = MT, NTH = NW * 64;
     constexpr int XS = TM * 8 + 2;  // words per block of the qs: a pad of two, so that lanes on consecutive blocks write distinct banks
@@ -635,13 +710,29 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
     const int nbj = I >> 5, JG = (nbj + NW - 1) / NW;
     // workgroup id % 8 is the XCD: each takes a contiguous eighth of the (tile, act block group) units, so
     // the tiles of one expert, which read the same weights, run together behind one L2
-    const int n_units = (int)(tiles[0] >> 18) * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
+    __shared__ __align__(16) int scnt[SCAN ? NW : 1][256], stok[SCAN ? NW : 1][MT];
+    TileScan sc;
+    const int n_tiles = SCAN ? sc.count(ids, P, E, scnt[wave]) : (int)(tiles[0] >> 18);
+    const int n_units = n_tiles * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
     const int unit = ((int)blockIdx.x & 7) * per + ur;
     if (ur >= per || unit >= n_units) return;
-    const uint32_t v0 = tiles[unit / JG];
-    const int jg = unit % JG, g = (int)(v0 >> 8) & 1023, c0 = (int)(v0 & 255) * MT;
-    const int e = meta[1 + g], s0 = meta[1 + E + g], nt = min(TM, meta[1 + 2 * E + g] - c0);
-    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
+    const int jg = unit % JG;
+    int e, c0, s0 = 0, nt;
+    if constexpr (SCAN) {
+        sc.find(unit / JG, P, stok[wave]);
+        e = sc.e;
+        c0 = sc.c0;
+        nt = min(TM, sc.n - c0);
+    } else {
+        const uint32_t v0 = tiles[unit / JG];
+        const int g = (int)(v0 >> 8) & 1023;
+        c0 = (int)(v0 & 255) * MT;
+        e = meta[1 + g];
+        s0 = meta[1 + E + g];
+        nt = min(TM, meta[1 + 2 * E + g] - c0);
+    }
+    auto pair = [&](int tt) __attribute__((always_inline)) { return SCAN ? stok[wave][tt] : plist[s0 + c0 + tt]; };
     const int jw = jg * NW + wave, j = min(jw, nbj - 1);
     // LDS: the tokens' q8 words [NH][4 lane groups][TM] (g, g+4) | [NH][TM] d / 16 | the waves' slice scales
     uint32_t* xq = reinterpret_cast<uint32_t*>(lds);
@@ -655,7 +746,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
             const int i = r * NTH + t, tt = i / NH, b = i - tt * NH;
             if (tt < nt) {
                 const uint2* src =
-                    reinterpret_cast<const uint2*>(q8x + ((int64_t)(plist[s0 + c0 + tt] / K) * NB + h * NH + b) * Q8_BLK);
+                    reinterpret_cast<const uint2*>(q8x + ((int64_t)(pair(tt) / K) * NB + h * NH + b) * Q8_BLK);
 #pragma unroll
                 for (int k = 0; k < 5; ++k) st[r][k] = src[k];
             }
@@ -676,6 +767,14 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
         }
     };
     load_act(0);
+    if (SCAN && jg == 0) {  // this tile's record, and the number of tiles
+        if (t < MT / 2) {
+            const uint32_t a = stok[0][min(2 * t, nt - 1)], b = stok[0][min(2 * t + 1, nt - 1)];
+            trec[unit / JG * TREC + 1 + t] = a | b << 16;
+        }
+        if (t == 0) trec[unit / JG * TREC] = (uint32_t)e | (uint32_t)nt << 16;
+        if (t == 0 && unit == 0) tiles[0] = tile_entry(n_tiles, 0, 0);
+    }
     const uint8_t* T = bank + (int64_t)e * expert_bytes + (int64_t)j * NB * 1152;
     const __amdgpu_buffer_rsrc_t rs = buf_rsrc(T, NB * 128), rw = buf_rsrc(T + NB * 128, NB * 1024);
     const uint32_t vw16 = lg * 256 + li * 16;
@@ -738,7 +837,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
                         for (int v = 0; v < 4; ++v) {
                             const int rr = 16 * m + 4 * lg + v;
                             const int row = rr < 32 ? j * 32 + rr : I + j * 32 + (rr - 32);
-                            rec[((int64_t)plist[s0 + c0 + slot] * 2 * I + row) * NB + s * BPW + b] = d[m][v] >> 4;
+                            rec[((int64_t)pair(slot) * 2 * I + row) * NB + s * BPW + b] = d[m][v] >> 4;
                         }
                 }
 #pragma unroll
@@ -765,7 +864,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
     }
     slice(7, std::true_type{});
     if (KH > 1 && jw >= nbj) return;
-    const int q = s0 + c0 + slot, p = plist[q];
+    const int p = pair(slot), q = SCAN ? p : s0 + c0 + slot;
     const bool ok = li < nt;
     const float isc = in_scale ? in_scale[p / K] : 1.0f;
     float a[8];
@@ -827,21 +926,33 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(const uint8_t* __r
 // an expert's tokens, rereading the weights for each 16: 512 tokens of the
 // Gemma shape 104 us, 173 zipf-skewed 93, 64 tokens 47; now 57, 31 and 33
 // (143 MB of weights, 4.4 TB/s).
-template <int NKB, int NW, bool LANES, bool REC>
+template <int NKB, int NW, bool LANES, bool REC, bool SCAN>
 __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
     const uint8_t* __restrict__ bank, int64_t expert_bytes, int64_t gu_bytes, const int32_t* __restrict__ meta,
     const uint32_t* __restrict__ tiles, const int32_t* __restrict__ plist, const uint8_t* __restrict__ q8m, int P,
-    float* ydn, int H, int I, int E, int32_t* rec) {
+    float* ydn, int H, int I, int E, int32_t* rec, const uint32_t* __restrict__ trec) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int NTH = NW * 64, NC = LANES ? 4 : 1, NBUF = 2;
     const int nbj = I >> 5, dn_tile = nbj * 288, RG = H / 64, JG = (RG + NW - 1) / NW;
     const int n_units = (int)(tiles[0] >> 18) * JG, per = (n_units + 7) >> 3, ur = (int)blockIdx.x >> 3;
     const int unit = ((int)blockIdx.x & 7) * per + ur;  // as k_mfma_gu_tok's
     if (ur >= per || unit >= n_units) return;
-    const uint32_t v0 = tiles[unit / JG];
-    const int g = (int)(v0 >> 8) & 1023, c0 = (int)(v0 & 255) * MT;
-    const int e = meta[1 + g], s0 = meta[1 + E + g], nt = min(MT, meta[1 + 2 * E + g] - c0);
+    int e, q0 = 0, nt;
+    const uint16_t* tp = nullptr;  // SCAN: the tile's pairs, which are also their positions in q8m
+    if constexpr (SCAN) {
+        const uint32_t* tr = trec + unit / JG * TREC;
+        e = (int)(tr[0] & 0xFFFF);
+        nt = (int)(tr[0] >> 16);
+        tp = reinterpret_cast<const uint16_t*>(tr + 1);
+    } else {
+        const uint32_t v0 = tiles[unit / JG];
+        const int g = (int)(v0 >> 8) & 1023, c0 = (int)(v0 & 255) * MT;
+        e = meta[1 + g];
+        q0 = meta[1 + E + g] + c0;
+        nt = min(MT, meta[1 + 2 * E + g] - c0);
+    }
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
+    const int qt = SCAN ? (int)tp[li] : q0 + min(li, nt - 1);  // slot li's position (past the tile: the last token's, never written out)
     const int rw0 = (unit % JG) * NW + wave, rg = min(rw0, RG - 1);  // this wave's 64 rows
     // LDS: the tokens' act words [nbj][4][MT] (g, g+4) | [nbj][MT] d / 16 | the waves' scales [4][nbj][16] f16
     uint2* xq = reinterpret_cast<uint2*>(lds);
@@ -866,14 +977,14 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
         uint2 w[R];
         float dv[RD];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {  // slots past the tile: the last token again, never written out
-            const int i = r * NTH + t, tt = min(i & 15, nt - 1);
-            if (i < nbj * 64) w[r] = q2[(int64_t)(i >> 4) * P + s0 + c0 + tt];
+        for (int r = 0; r < R; ++r) {  // item i: slot i % 16 = li, as NTH is a multiple of 16
+            const int i = r * NTH + t;
+            if (i < nbj * 64) w[r] = q2[(int64_t)(i >> 4) * P + qt];
         }
 #pragma unroll
         for (int r = 0; r < RD; ++r) {
-            const int i = r * NTH + t, tt = min(i & 15, nt - 1);
-            if (i < nbj * 16) dv[r] = __uint_as_float(q2[(int64_t)P * nbj * 4 + (int64_t)(i >> 4) * P + s0 + c0 + tt].x) * 0.0625f;
+            const int i = r * NTH + t;
+            if (i < nbj * 16) dv[r] = __uint_as_float(q2[(int64_t)P * nbj * 4 + (int64_t)(i >> 4) * P + qt].x) * 0.0625f;
         }
 #pragma unroll
         for (int r = 0; r < R; ++r)
@@ -890,7 +1001,7 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
     float acc[NC][4][4];
 #pragma unroll
     for (int i = 0; i < NC * 16; ++i) acc[i >> 4][i >> 2 & 3][i & 3] = 0.0f;
-    const int p = plist[s0 + c0 + min(li, nt - 1)];
+    const int p = SCAN ? qt : plist[qt];
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
         if (kb + NBUF - 1 < NKB) load(kb + NBUF - 1, (kb + NBUF - 1) % NBUF);
@@ -1225,7 +1336,14 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // every expert on the dot4 kernels, routing already in ids: the dot4
     // workgroups find their expert's pairs themselves (no grouping launch)
     const bool scan = !topk_in && n_mfma > P && P <= SCAN_MAX;
-    if (!scan) {
+    const bool rec = ctx->rec_gu && ctx->rec_dn;
+    // Every expert on the token-tile MFMA kernels: up to TILE_SCAN pairs their waves find the tiles themselves, which
+    // costs them less than the grouping launch: 16 tokens of the Gemma shape with uniform / zipf-skewed routing 82.3 /
+    // 55.4 us a layer against 85.9 / 59.5, 20 tokens 97.2 / 60.9 against 100.2 / 64.5, 63 tokens 119.4 / 85.8 against
+    // 121.7 / 86.7, 64 tokens as much.
+    const bool tscan = !topk_in && n_mfma == 1 && P <= TILE_SCAN && E <= 256 && nbj <= 32 && !rec && !dbg_act &&
+                       (H != 2816 || P < 9 * E);
+    if (!scan && !tscan) {
         hipLaunchKernelGGL(topk_in ? k_group_pairs<true> : k_group_pairs<false>, dim3(1), dim3(1024), 0, s,
                            (const int32_t*)ids, P, E, n_mfma, w.meta, w.plist, w.ppos, (const float*)w.logits,
                            expert_scale, ids, wts, K);
@@ -1242,7 +1360,6 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // the instantiations that store every int32 block dot
     int32_t* rgu = ctx->rec_gu;
     int32_t* rdn = ctx->rec_dn;
-    const bool rec = rgu && rdn;
     if (dot4) {
         const size_t lds_gu = (size_t)NT * nb * 40 + sizeof(float) * (GW * NT * 64 + NT * 64 + NT * 32) + 4 * NT * 10;
         auto kern = scan ? (H == 2816 ? (rec ? k_grouped_gu<11, true, true> : k_grouped_gu<11, false, true>)
@@ -1258,8 +1375,9 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         auto gate_up = [&](auto kern, int nw, int kh) {
             const size_t lds_mg = (size_t)nb / kh * ((MT * 8 + 2) * 4 + MT * 4) + (size_t)nw * nb / 8 * 128;
             hipLaunchKernelGGL(kern, dim3(((nbj + nw - 1) / nw * n_tiles + 7) / 8 * 8), dim3(nw * 64), lds_mg, s,
-                               (const uint8_t*)bank, eb, (const int32_t*)w.meta, (const uint32_t*)w.ppos,
-                               (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, I, E, K, P, rgu);
+                               (const uint8_t*)bank, eb, (const int32_t*)w.meta, (uint32_t*)w.ppos,
+                               (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, I, E, K, P, rgu,
+                               (const int32_t*)ids, (uint32_t*)w.q8a);
         };
         // Two forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
         // for all 128 of the Gemma shape), and small workgroups that hold half of the tokens' rows at a time
@@ -1268,11 +1386,15 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         // waves share one staging of whole rows, two workgroups to a CU: 512 tokens 118-126 us against 137,
         // 173 zipf-skewed tokens 67 against 70; at 10 pairs per expert 74 against 80 (zipf-skewed 67, 71).
         if (H == 2816 && P < 9 * E)
-            gate_up(rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true> : k_mfma_gu_tok<11, 4, 3, 8, 2, false>, 4, 2);
+            gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 8, 2, false, true>
+                    : rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true, false>
+                          : k_mfma_gu_tok<11, 4, 3, 8, 2, false, false>, 4, 2);
         else if (H == 2816)
-            gate_up(rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true> : k_mfma_gu_tok<11, 8, 4, 6, 1, false>, 8, 1);
+            gate_up(rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false> : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false>, 8, 1);
         else
-            gate_up(rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true> : k_mfma_gu_tok<16, 16, 4, 6, 1, false>, 16, 1);
+            gate_up(tscan ? k_mfma_gu_tok<16, 16, 4, 6, 1, false, true>
+                    : rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true, false>
+                          : k_mfma_gu_tok<16, 16, 4, 6, 1, false, false>, 16, 1);
         if ((rc = launch_status("moe_layer_grouped/gate_up_mfma"))) return rc;
         if (dbg_act) {  // the debug copy below reads q8a's pair rows
             hipLaunchKernelGGL(k_q8m_rows, dim3(64, (unsigned)gbig), dim3(256), 0, s,
@@ -1298,15 +1420,18 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         if (nbj <= 32) {
             constexpr int NW = 4;
             const size_t lds_md = (size_t)nbj * (576 + NW * 128);
-            auto pick = [&](auto ln) {
-                constexpr bool LN = decltype(ln)::value;
-                return nbj <= 24 ? (rec ? k_mfma_down_tok<6, NW, LN, true> : k_mfma_down_tok<6, NW, LN, false>)
-                                 : (rec ? k_mfma_down_tok<8, NW, LN, true> : k_mfma_down_tok<8, NW, LN, false>);
+            auto form = [&](auto ln, auto rc, auto sn) {
+                constexpr bool LN = decltype(ln)::value, RC = decltype(rc)::value, SN = decltype(sn)::value;
+                return nbj <= 24 ? k_mfma_down_tok<6, NW, LN, RC, SN> : k_mfma_down_tok<8, NW, LN, RC, SN>;
             };
-            auto kern = lanes ? pick(std::true_type{}) : pick(std::false_type{});
+            constexpr std::true_type T{};
+            constexpr std::false_type F{};
+            auto pick = [&](auto ln) { return tscan ? form(ln, F, T) : rec ? form(ln, T, F) : form(ln, F, F); };
+            auto kern = lanes ? pick(T) : pick(F);
             hipLaunchKernelGGL(kern, dim3(((H / 64 + NW - 1) / NW * n_tiles + 7) / 8 * 8), dim3(NW * 64), lds_md, s,
                                (const uint8_t*)bank, eb, gu_bytes, (const int32_t*)w.meta, (const uint32_t*)w.ppos,
-                               (const int32_t*)w.plist, (const uint8_t*)w.q8m, P, w.ydn, H, I, E, rdn);
+                               (const int32_t*)w.plist, (const uint8_t*)w.q8m, P, w.ydn, H, I, E, rdn,
+                               (const uint32_t*)w.q8a);
         } else {  // long rows: DRT tiles per workgroup, 8 K slices of 56 (rows up to 448 blocks) or 64 blocks
             constexpr int DRT = 4;
             const size_t lds_md = std::max((size_t)DRT * nbj * 32, sizeof(float) * GW * DRT * 16 * MT);

@@ -123,6 +123,9 @@ def test_routing_of_many_seqs_matches_few(gemv, hidden, E, K, B, norm):
     (4096, 1024, 9, 3, 11),    # 32 act blocks
     (4096, 32, 40, 1, 159),    # one act block, three of the four chains empty
     (2816, 96, 3, 1, 11),
+    (2816, 96, 256, 8, 64),    # the most pairs and experts of a layer without a grouping launch
+    (2816, 96, 257, 8, 64),    # more experts
+    (4096, 96, 200, 3, 171),   # more pairs
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, inter, E, K, B, norm):
