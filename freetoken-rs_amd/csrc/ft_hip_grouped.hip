@@ -695,7 +695,11 @@ struct TileScan {
 // matrix cores, 24 for operands and 10 for the GELU epilogue); for few the
 // weights (64 tokens: 285 MB in 63 us, 4.5 TB/s). Blocks are consumed one at a
 // time (sched_barrier), else the registers of a whole slice's dots spill.
-template <int BPW, int NW, int WPE, int D, int KH, bool REC, bool SCAN>
+// KS, for launches of few units: a workgroup is one act block, its 8 waves a
+// slice each, and the first adds their sums in slice order, the same bits. The
+// chain of a wave is an eighth as long: 16 tokens over 8 experts of H 4096, I 1024
+// 104 -> 41 us a layer, of H 2816, I 704 45 -> 34.
+template <int BPW, int NW, int WPE, int D, int KH, bool REC, bool SCAN, bool KS>
 __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
     const uint8_t* __restrict__ bank, int64_t expert_bytes, const int32_t* __restrict__ meta, uint32_t* tiles,
     const int32_t* __restrict__ plist, const uint8_t* __restrict__ q8x, uint8_t* q8m, float* dbg_gu,
@@ -707,7 +711,8 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
     constexpr int NH = NB / KH, SH = 8 / KH;  // blocks and slices per staging of the tokens' rows
     constexpr int R = (TM * NH + NTH - 1) / NTH;  // (token, block) items staged per thread
     constexpr int SW = BPW * 128;   // bytes of a slice's scales
-    const int nbj = I >> 5, JG = (nbj + NW - 1) / NW;
+    static_assert(!KS || (NW == 8 && KH == 1), "a wave per slice");
+    const int nbj = I >> 5, JG = KS ? nbj : (nbj + NW - 1) / NW;
     // workgroup id % 8 is the XCD: each takes a contiguous eighth of the (tile, act block group) units, so
     // the tiles of one expert, which read the same weights, run together behind one L2
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
@@ -733,7 +738,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
         nt = min(TM, meta[1 + 2 * E + g] - c0);
     }
     auto pair = [&](int tt) __attribute__((always_inline)) { return SCAN ? stok[wave][tt] : plist[s0 + c0 + tt]; };
-    const int jw = jg * NW + wave, j = min(jw, nbj - 1);
+    const int jw = KS ? jg : jg * NW + wave, j = min(jw, nbj - 1), sl0 = KS ? wave : 0;  // sl0: the wave's first slice
     // LDS: the tokens' q8 words [NH][4 lane groups][TM] (g, g+4) | [NH][TM] d / 16 | the waves' slice scales
     uint32_t* xq = reinterpret_cast<uint32_t*>(lds);
     float* xd = reinterpret_cast<float*>(lds + (size_t)NH * XS * 4);
@@ -783,9 +788,9 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
         ss[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, s * SW, 0);
         ss[1] = __builtin_amdgcn_raw_buffer_load_b128(rs, min(1024 + lane * 16, SW - 16), s * SW, 0);
     };
-    load_scales(0);
+    load_scales(sl0);
 #pragma unroll
-    for (int b = 0; b < D; ++b) aw[b] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, b * 1024, 0);
+    for (int b = 0; b < D; ++b) aw[b] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, (sl0 * BPW + b) * 1024, 0);
     store_act();
     __syncthreads();
     if (KH == 1 && jw >= nbj) return;
@@ -852,17 +857,41 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
 #pragma unroll
             for (int v = 0; v < 4; ++v) tot[m][v] = tot[m][v] + acc[m][v];
     };
-#pragma unroll 1
-    for (int s = 0; s < 7; ++s) {
-        if (KH > 1 && s == SH) {  // the rest of the tokens' rows, once every wave is done with the first part
-            load_act(1);
-            __syncthreads();
-            store_act();
-            __syncthreads();
+    if constexpr (KS) {
+        slice(wave, std::true_type{});
+        // the other waves' slice sums through LDS (over the tokens' rows), added in slice order by the first
+        float4* part = reinterpret_cast<float4*>(lds);
+        auto at = [&](int s, int m) { return (s * 64 + lane) * 4 + ((m + (lane >> 1)) & 3); };
+        __syncthreads();
+        if (wave > 0) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) part[at(wave, m)] = make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]);
         }
-        slice(s, std::false_type{});
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int s = 1; s < 8; ++s)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const float4 v = part[at(s, m)];
+                tot[m][0] = tot[m][0] + v.x;
+                tot[m][1] = tot[m][1] + v.y;
+                tot[m][2] = tot[m][2] + v.z;
+                tot[m][3] = tot[m][3] + v.w;
+            }
+    } else {
+#pragma unroll 1
+        for (int s = 0; s < 7; ++s) {
+            if (KH > 1 && s == SH) {  // the rest of the tokens' rows, once every wave is done with the first part
+                load_act(1);
+                __syncthreads();
+                store_act();
+                __syncthreads();
+            }
+            slice(s, std::false_type{});
+        }
+        slice(7, std::true_type{});
     }
-    slice(7, std::true_type{});
     if (KH > 1 && jw >= nbj) return;
     const int p = pair(slot), q = SCAN ? p : s0 + c0 + slot;
     const bool ok = li < nt;
@@ -1320,19 +1349,25 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // groups of >= n_mfma tokens take the MFMA tile kernels, the others the
     // dot4 kernels; rows longer than 32 blocks (I > 1024) only the former.
     // Automatic (0): every group on one family, MFMA from 2/3 of a pair per
-    // expert on (its grouping, gate|up and down launches against dot4's two, on
-    // the Gemma shape with uniform / zipf-skewed routing: 8 tokens 58.7 / 42.0
-    // us against 51.0 / 45.4, 11 tokens 60.8 / 42.9 against 60.7 / 60.1, 16
-    // tokens 71.3 / 45.7 against 76.9 / 79.2, 63 tokens 101 / 67 against 146 /
-    // 246: dot4's cost grows with an expert's tokens)
+    // expert on (layers of the Gemma shape with uniform / zipf-skewed routing, MFMA
+    // against dot4: 8 tokens 65 / 48 us against 60 / 48, 11 tokens 71 / 54 against 73 /
+    // 60, 16 tokens 82 / 52 against 87 / 83, 24 tokens 101 / 60 against 103 / 111, 63
+    // tokens 119 / 86 against 160 / 252: dot4's cost grows with an expert's tokens),
+    // and, below 4, only from 64 pairs (H 2816) or 96 (H 4096) on: fewer leave the
+    // MFMA kernels' larger units too few (32 experts of I 704: 48 pairs 50 / 47 against
+    // 47 / 54, 64 pairs 50 / 48 against 52 / 62; 64 experts of H 4096, I 1024: 64 pairs
+    // 112 / 106 against 98 / 90, 96 pairs 120 / 112 against 118 / 115, 128 pairs 124 /
+    // 115 against 135 / 136)
     int n_mfma = ctx->grouped_mfma_min;
-    if (n_mfma <= 0) n_mfma = 3LL * P >= 2 * n_experts ? 1 : std::numeric_limits<int>::max();
+    const bool sparse = P < 4LL * n_experts;
+    if (n_mfma <= 0)
+        n_mfma = sparse && (3LL * P < 2 * n_experts || P < (H == 2816 ? 64 : 96)) ? std::numeric_limits<int>::max() : 1;
     if (nbj > 32) n_mfma = 1;
     // Automatic, below 4 pairs per expert: the down sums in the dot4 kernels' order, so that where the line above
     // lies in this range shows in no output bit (another order of 22 block sums moves q8 quants of the layers that
     // follow: 3e-4 of the state after four layers). From there on, and where the caller splits the experts, one chain
     // in block order, the faster form.
-    const bool lanes = ctx->grouped_mfma_min <= 0 && P < 4LL * n_experts;
+    const bool lanes = ctx->grouped_mfma_min <= 0 && sparse;
     // every expert on the dot4 kernels, routing already in ids: the dot4
     // workgroups find their expert's pairs themselves (no grouping launch)
     const bool scan = !topk_in && n_mfma > P && P <= SCAN_MAX;
@@ -1341,8 +1376,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // costs them less than the grouping launch: 16 tokens of the Gemma shape with uniform / zipf-skewed routing 82.3 /
     // 55.4 us a layer against 85.9 / 59.5, 20 tokens 97.2 / 60.9 against 100.2 / 64.5, 63 tokens 119.4 / 85.8 against
     // 121.7 / 86.7, 64 tokens as much.
-    const bool tscan = !topk_in && n_mfma == 1 && P <= TILE_SCAN && E <= 256 && nbj <= 32 && !rec && !dbg_act &&
-                       (H != 2816 || P < 9 * E);
+    const bool tscan = !topk_in && n_mfma == 1 && P <= TILE_SCAN && E <= 256 && nbj <= 32 && !rec && !dbg_act;
     if (!scan && !tscan) {
         hipLaunchKernelGGL(topk_in ? k_group_pairs<true> : k_group_pairs<false>, dim3(1), dim3(1024), 0, s,
                            (const int32_t*)ids, P, E, n_mfma, w.meta, w.plist, w.ppos, (const float*)w.logits,
@@ -1372,29 +1406,45 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         if ((rc = launch_status("moe_layer_grouped/gate_up"))) return rc;
     }
     if (mfma) {
-        auto gate_up = [&](auto kern, int nw, int kh) {
+        auto gate_up = [&](auto kern, int nw, int kh, int jpw) {
             const size_t lds_mg = (size_t)nb / kh * ((MT * 8 + 2) * 4 + MT * 4) + (size_t)nw * nb / 8 * 128;
-            hipLaunchKernelGGL(kern, dim3(((nbj + nw - 1) / nw * n_tiles + 7) / 8 * 8), dim3(nw * 64), lds_mg, s,
+            hipLaunchKernelGGL(kern, dim3(((nbj + jpw - 1) / jpw * n_tiles + 7) / 8 * 8), dim3(nw * 64), lds_mg, s,
                                (const uint8_t*)bank, eb, (const int32_t*)w.meta, (uint32_t*)w.ppos,
                                (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, I, E, K, P, rgu,
                                (const int32_t*)ids, (uint32_t*)w.q8a);
         };
-        // Two forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
+        // Three forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
         // for all 128 of the Gemma shape), and small workgroups that hold half of the tokens' rows at a time
         // (36 KB of LDS, 3 to a CU) spread them best over the CUs: 64 tokens 63 us against 73 for the other
         // form, 127 tokens 64 against 73 (zipf-skewed 55 against 65). More tokens: the VALU bounds it, and 8
         // waves share one staging of whole rows, two workgroups to a CU: 512 tokens 118-126 us against 137,
         // 173 zipf-skewed tokens 67 against 70; at 10 pairs per expert 74 against 80 (zipf-skewed 67, 71).
-        if (H == 2816 && P < 9 * E)
-            gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 8, 2, false, true>
-                    : rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true, false>
-                          : k_mfma_gu_tok<11, 4, 3, 8, 2, false, false>, 4, 2);
+        // Few (tile, act block) units for the chip's 256 CUs: a wave that walks whole rows takes 25 us (H 2816) or
+        // 80 (H 4096, 16 to a CU) however few they are, so the 8 slices of a row go to 8 waves. Layers, that form
+        // against the other, uniform / zipf-skewed routing, by this bound on the units: H 2816 (I 704) 550 units 43 /
+        // 43 us against 58 / 59, 704 (under 9 pairs per expert) 42 / 39 against 47 / 46, 792 53 / 42 against 50 / 48,
+        // 902 58 / 56 against 55 / 56, 1056 (over) 64 / 64 against 67 / 67, 1760 94 / 95 against 80 / 81; H 4096
+        // (I 1024) 768 73 against 113, 1536 100 / 111 against 119 / 123, 2048 149 / 164 against 128 / 131.
+        const int64_t units = (int64_t)nbj * n_tiles;
+        const bool ks = !rec && units <= (H == 2816 ? (P < 9 * E ? 3 : 4) : 6) * 256;
+        if (H == 2816 && ks)
+            gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, true>
+                          : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false, true>, 8, 1, 1);
+        else if (ks)
+            gate_up(tscan ? k_mfma_gu_tok<16, 8, 2, 16, 1, false, true, true>
+                          : k_mfma_gu_tok<16, 8, 2, 16, 1, false, false, true>, 8, 1, 1);
+        else if (H == 2816 && P < 9 * E)
+            gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 8, 2, false, true, false>
+                    : rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true, false, false>
+                          : k_mfma_gu_tok<11, 4, 3, 8, 2, false, false, false>, 4, 2, 4);
         else if (H == 2816)
-            gate_up(rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false> : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false>, 8, 1);
+            gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, false>
+                    : rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false, false>
+                          : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false, false>, 8, 1, 8);
         else
-            gate_up(tscan ? k_mfma_gu_tok<16, 16, 4, 6, 1, false, true>
-                    : rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true, false>
-                          : k_mfma_gu_tok<16, 16, 4, 6, 1, false, false>, 16, 1);
+            gate_up(tscan ? k_mfma_gu_tok<16, 16, 4, 6, 1, false, true, false>
+                    : rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true, false, false>
+                          : k_mfma_gu_tok<16, 16, 4, 6, 1, false, false, false>, 16, 1, 16);
         if ((rc = launch_status("moe_layer_grouped/gate_up_mfma"))) return rc;
         if (dbg_act) {  // the debug copy below reads q8a's pair rows
             hipLaunchKernelGGL(k_q8m_rows, dim3(64, (unsigned)gbig), dim3(256), 0, s,

@@ -24,6 +24,10 @@ DEV = "cuda:0"
     (2816, 1024, [33, 0, 0, 0, 0, 0, 0, 38]),      # 71 pairs: just under, two experts only
     (2816, 416, [72, 0, 0, 0, 0, 0, 0, 0]),        # 72 pairs: on the line, one expert
     (4096, 96, [17, 0, 1, 16, 0, 0, 0, 33]),
+    # (these few units take the form of a slice per wave; enough of them for the forms of an act block per wave)
+    (2816, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 1] * 9 + [7]),          # 4 waves
+    (2816, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 17] * 9 + [16]),        # 8: over 9 pairs per expert
+    (4096, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 4, 3, 1] * 8 + [48]),   # 16
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_token_tiles_match_dot4(gemv, hidden, inter, counts, norm):
@@ -126,6 +130,7 @@ def test_routing_of_many_seqs_matches_few(gemv, hidden, E, K, B, norm):
     (2816, 96, 256, 8, 64),    # the most pairs and experts of a layer without a grouping launch
     (2816, 96, 257, 8, 64),    # more experts
     (4096, 96, 200, 3, 171),   # more pairs
+    (2816, 96, 40, 4, 30),
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, inter, E, K, B, norm):
@@ -159,3 +164,31 @@ def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, 
     finally:
         gemv.set_input_norm(0)
         gemv.set_grouped_mfma_min(0)
+
+
+@pytest.mark.parametrize("hidden,inter,E,K,B", [(2816, 992, 40, 8, 48), (2816, 96, 40, 8, 48), (4096, 992, 40, 4, 100),
+                                                (4096, 96, 40, 4, 41), (2816, 992, 100, 4, 128)])
+def test_tiles_found_without_the_grouping_launch(gemv, hidden, inter, E, K, B):
+    """A call that asks for the act blocks goes through the grouping launch; the
+    output bits are those of the call that does not."""
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 80), ft_hip.LAYOUT_Q4R)
+    src = torch.empty(E * eb, dtype=torch.uint8, device=DEV)
+    for e in range(E):
+        gemv.gen_q4_rows(7000 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(8000 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    rng = np.random.default_rng(hidden + inter + B)
+    x = torch.from_numpy(rng.standard_normal((B, hidden)).astype(np.float32)).to(DEV)
+    w = torch.from_numpy((rng.standard_normal((E, hidden)) * 0.02).astype(np.float32)).to(DEV)
+    bias = torch.linspace(2, -2, E, device=DEV)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+    got = []
+    for act in (None, torch.zeros((B * K, inter // 32, 40), dtype=torch.uint8, device=DEV)):
+        out = torch.zeros_like(x)
+        ids = torch.zeros(B * K, dtype=torch.int32, device=DEV)
+        wts = torch.zeros(B * K, dtype=torch.float32, device=DEV)
+        gemv.moe_layer_grouped(x, out, B, hidden, inter, E, K, w, bias, None, bank, ids, wts, ws, None, act)
+        torch.cuda.synchronize()
+        got.append(out.cpu().numpy().view(np.uint32))
+    assert np.array_equal(got[0], got[1])
