@@ -176,11 +176,15 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
     int ex[MAX_PAIRS / 1024], at[MAX_PAIRS / 1024];
 #pragma unroll
     for (int i = 0; i < MAX_PAIRS / 1024; ++i) {
+        if (i * 1024 >= P) break;
         const int p = i * 1024 + t;
         ex[i] = p < P ? min(max(pid(p), 0), E - 1) : 0;
     }
 #pragma unroll
-    for (int i = 0; i < MAX_PAIRS / 1024; ++i) at[i] = i * 1024 + t < P ? atomicAdd(&cnt[ex[i]], 1) : 0;
+    for (int i = 0; i < MAX_PAIRS / 1024; ++i) {
+        if (i * 1024 >= P) break;  // uniform
+        if (i * 1024 + t < P) at[i] = atomicAdd(&cnt[ex[i]], 1);
+    }
     __syncthreads();
     // inclusive prefix sums of counts and of "active" / "big" flags (E <=
     // 1024): within each wavefront by shuffles, then each thread adds the
@@ -232,7 +236,7 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < MAX_PAIRS / 1024; ++i)
+    for (int i = 0; i < MAX_PAIRS / 1024 && i * 1024 < P; ++i)
         if (i * 1024 + t < P) plist[scan[ex[i]] - cnt[ex[i]] + at[i]] = i * 1024 + t;
     // the tile list (every tile holds a pair, so P entries suffice)
     for (int k = 0; k < my_tiles; ++k) ppos[vt - my_tiles + k] = (int32_t)tile_entry(n_tiles, big[t] - 1, k * MT);
