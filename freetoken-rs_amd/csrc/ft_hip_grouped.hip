@@ -564,14 +564,14 @@ __device__ __forceinline__ long nib_op(uint32_t w) {
     return (long)(((uint64_t)((w >> 4) & 0x0F0F0F0Fu) << 32) | (w & 0x0F0F0F0Fu));
 }
 
-// The same, signed: 16 * (q - 8) as bytes (the nibble in the byte's high half,
-// its top bit flipped), so D is 16 times the block dot, the accumulator starts
-// at zero and qsum is not needed. The kernels that use it take d8 / 16, exact,
-// so a product of scales and every sum has the bits it has with the plain dot
-// (short of products below 2^-122, which are subnormal then).
-__device__ __forceinline__ long nib_op16(uint32_t w) {
-    const uint32_t lo = ((w << 4) & 0xF0F0F0F0u) ^ 0x80808080u, hi = (w & 0xF0F0F0F0u) ^ 0x80808080u;
-    return (long)(((uint64_t)hi << 32) | lo);
+// -8 * qsum of each token's block in the lanes and rows of a 16x16 tile, the
+// accumulators' start for nib_op's unsigned nibbles: the block against rows of
+// -8, one more instruction on the matrix cores (which the token-tile kernels leave idle
+// most of the time) where a broadcast takes four on the VALU and qsum in LDS.
+// (Signed operands 16 * (q - 8) and d8 / 16 need no start, but then a scale
+// product below 2^-122 is rounded as a subnormal.)
+__device__ __forceinline__ v4i start_sums(long bop) {
+    return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)0xF8F8F8F8F8F8F8F8ull, bop, v4i{0, 0, 0, 0}, 0, 0, 0);
 }
 
 // d4 * d8 of a 16x16 tile's (row, token) pairs, each rounded once as by
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
     }
     auto pair = [&](int tt) __attribute__((always_inline)) { return SCAN ? stok[wave][tt] : plist[s0 + c0 + tt]; };
     const int jw = KS ? jg : jg * NW + wave, j = min(jw, nbj - 1), sl0 = KS ? wave : 0;  // sl0: the wave's first slice
-    // LDS: the tokens' q8 words [NH][4 lane groups][TM] (g, g+4) | [NH][TM] d / 16 | the waves' slice scales
+    // LDS: the tokens' q8 words [NH][4 lane groups][TM] (g, g+4) | [NH][TM] d | the waves' slice scales
     uint32_t* xq = reinterpret_cast<uint32_t*>(lds);
     float* xd = reinterpret_cast<float*>(lds + (size_t)NH * XS * 4);
     uint8_t* scl = lds + (size_t)NH * (XS * 4 + TM * 4) + wave * SW;
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
                 *reinterpret_cast<uint2*>(q + TM * 2) = make_uint2(st[r][1].y, st[r][3].y);
                 *reinterpret_cast<uint2*>(q + TM * 4) = make_uint2(st[r][2].x, st[r][4].x);
                 *reinterpret_cast<uint2*>(q + TM * 6) = make_uint2(st[r][2].y, st[r][4].y);
-                xd[b * TM + tt] = __uint_as_float(st[r][0].x) * 0.0625f;
+                xd[b * TM + tt] = __uint_as_float(st[r][0].x);
             }
         }
     };
@@ -831,13 +831,14 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
             if (b + D < BPW || !last)  // the block D ahead
                 aw[(b + D) % BPW] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw16, (s * BPW + b + D) * 1024, 0);
             const long bop = (long)(((uint64_t)q.y << 32) | q.x);
+            const v4i c8 = start_sums(bop);
             v4i d[4];
             v4f sp[4];
 #pragma unroll
             for (int m = 0; m < 4; ++m) sp[m] = scale_products(dw[m], ad);
 #pragma unroll
             for (int m = 0; m < 4; ++m)
-                d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op16(w[m]), bop, v4i{0, 0, 0, 0}, 0, 0, 0);
+                d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op(w[m]), bop, c8, 0, 0, 0);
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 if constexpr (REC) {  // test record: the (row, token) blocks' int32 dots
@@ -846,7 +847,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
                         for (int v = 0; v < 4; ++v) {
                             const int rr = 16 * m + 4 * lg + v;
                             const int row = rr < 32 ? j * 32 + rr : I + j * 32 + (rr - 32);
-                            rec[((int64_t)pair(slot) * 2 * I + row) * NB + s * BPW + b] = d[m][v] >> 4;
+                            rec[((int64_t)pair(slot) * 2 * I + row) * NB + s * BPW + b] = d[m][v];
                         }
                 }
 #pragma unroll
@@ -987,7 +988,7 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, li = t & 15, lg = lane >> 4;
     const int qt = SCAN ? (int)tp[li] : q0 + min(li, nt - 1);  // slot li's position (past the tile: the last token's, never written out)
     const int rw0 = (unit % JG) * NW + wave, rg = min(rw0, RG - 1);  // this wave's 64 rows
-    // LDS: the tokens' act words [nbj][4][MT] (g, g+4) | [nbj][MT] d / 16 | the waves' scales [4][nbj][16] f16
+    // LDS: the tokens' act words [nbj][4][MT] (g, g+4) | [nbj][MT] d | the waves' scales [4][nbj][16] f16
     uint2* xq = reinterpret_cast<uint2*>(lds);
     float* xd = reinterpret_cast<float*>(lds + (size_t)nbj * 512);
     uint8_t* scl = lds + (size_t)nbj * 576 + (size_t)wave * nbj * 128;
@@ -1017,7 +1018,7 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
 #pragma unroll
         for (int r = 0; r < RD; ++r) {
             const int i = r * NTH + t;
-            if (i < nbj * 16) dv[r] = __uint_as_float(q2[(int64_t)P * nbj * 4 + (int64_t)(i >> 4) * P + qt].x) * 0.0625f;
+            if (i < nbj * 16) dv[r] = __uint_as_float(q2[(int64_t)P * nbj * 4 + (int64_t)(i >> 4) * P + qt].x);
         }
 #pragma unroll
         for (int r = 0; r < R; ++r)
@@ -1055,6 +1056,7 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
                 const uint2 q = xq[(blk * 4 + lg) * MT + li];
                 const float ad = xd[blk * MT + li];
                 const long bop = (long)(((uint64_t)q.y << 32) | q.x);
+                const v4i c8 = start_sums(bop);
                 v4i d[4];
                 v4f sp[4];
 #pragma unroll
@@ -1064,14 +1066,14 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
                 }
 #pragma unroll
                 for (int m = 0; m < 4; ++m)
-                    d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op16(w[m][b]), bop, v4i{0, 0, 0, 0}, 0, 0, 0);
+                    d[m] = __builtin_amdgcn_mfma_i32_16x16x32_i8(nib_op(w[m][b]), bop, c8, 0, 0, 0);
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     if constexpr (REC) {  // test record: the (row, token) blocks' int32 dots
                         if (li < nt)
 #pragma unroll
                             for (int v = 0; v < 4; ++v)
-                                rec[((int64_t)p * H + rg * 64 + m * 16 + 4 * lg + v) * nbj + blk] = d[m][v] >> 4;
+                                rec[((int64_t)p * H + rg * 64 + m * 16 + 4 * lg + v) * nbj + blk] = d[m][v];
                     }
                     float(&a)[4] = acc[b % NC][m];
 #pragma unroll
@@ -1440,7 +1442,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         else if (H == 2816 && P < 9 * E)
             gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 8, 2, false, true, false>
                     : rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true, false, false>
-                          : k_mfma_gu_tok<11, 4, 3, 8, 2, false, false, false>, 4, 2, 4);
+                          : k_mfma_gu_tok<11, 4, 3, 7, 2, false, false, false>, 4, 2, 4);
         else if (H == 2816)
             gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, false>
                     : rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false, false>
