@@ -181,21 +181,21 @@ __device__ __forceinline__ float topk_softmax(const float* selv, const int* seli
     return w;
 }
 
-// Four blocks of a row, b, b+step, ...: their loads issued together (past the
+// N blocks of a row, b, b+step, ...: their loads issued together (past the
 // row's end its last block again, not used).
-template <int LAYOUT>
-struct Blocks4 {
-    float d4[4];
-    uint4 q[4];
+template <int LAYOUT, int N>
+struct Blocks {
+    float d4[N];
+    uint4 q[N];
     __device__ __forceinline__ void load(const uint8_t* wr, int b, int step, int nb, int qs_off) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) load_block<LAYOUT>(wr, min(b + step * u, nb - 1), qs_off, d4[u], q[u]);
+        for (int u = 0; u < N; ++u) load_block<LAYOUT>(wr, min(b + step * u, nb - 1), qs_off, d4[u], q[u]);
     }
     // the blocks below nb onto acc, in order
     template <bool REC>
     __device__ __forceinline__ float dots(float acc, int b, int step, int nb, const int* lds, int32_t* rec) const {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < N; ++u) {
             const int bb = b + step * u;
             const int* xb = lds + min(bb, nb - 1) * 10;
             const float d8 = __int_as_float(xb[0]);
@@ -209,15 +209,17 @@ struct Blocks4 {
 
 // One row's share of a lane: lane `sub` of the row's LPR takes blocks sub,
 // sub+LPR, ..., an fma chain in block order (four blocks' loads issued
-// together, the last one to four as well: a row is otherwise one load latency
-// per block). The caller sums the LPR lanes by xor 1, 2, 4 (, 8).
+// together, the last one to four as well, no more than there are: a row is
+// otherwise one load latency per block). The caller sums the LPR lanes by xor
+// 1, 2, 4 (, 8).
 template <int LAYOUT, int LPR = 8, bool REC = false>
 __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int nb, const int* lds,
                                                int32_t* rec = nullptr) {
     const int qs_off = (nb * 2 + 15) / 16 * 16;
     float acc = 0.0f;
     int b = sub;
-    for (; b + 3 * LPR < nb; b += 4 * LPR) {
+    const int full = LPR > 8 ? nb - 3 * LPR : nb - 4 * LPR + 1 + sub;  // up to 8 lanes: rounds all of them take whole
+    for (; b < full; b += 4 * LPR) {
         float d4[4];
         uint4 q[4];
 #pragma unroll
@@ -232,11 +234,16 @@ __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int n
         }
     }
     if constexpr (LPR <= 8) {
-        if (b < nb) {
-            Blocks4<LAYOUT> k;
+        auto tail = [&](auto n) __attribute__((always_inline)) {
+            Blocks<LAYOUT, decltype(n)::value> k;
             k.load(wr, b, LPR, nb, qs_off);
             acc = k.template dots<REC>(acc, b, LPR, nb, lds, rec);
-        }
+        };
+        const int left = (nb % (4 * LPR) + LPR - 1) / LPR;  // uniform
+        if (left == 4) tail(std::integral_constant<int, 4>{});
+        else if (left == 3) tail(std::integral_constant<int, 3>{});
+        else if (left == 2) tail(std::integral_constant<int, 2>{});
+        else if (left == 1) tail(std::integral_constant<int, 1>{});
     } else {  // long rows: the tail is a small part, and its code costs the loop above (large-expert stack 1 %)
         for (; b < nb; b += LPR) {
             float d4;
@@ -297,9 +304,9 @@ __device__ __forceinline__ float sum_row_lanes(float acc) {
 // rows of one entry: 8 lanes per row, lane s takes blocks s, s+8, ...; the
 // activation sits in LDS. REC: every block's int32 dot is also stored to
 // a.dots[e][row][block] (test record). Grid: (ceil(n_rows/32), n_entries).
-// SHORT (rows of up to 32 blocks): a lane's blocks are loaded before the
+// NBL > 0 (rows of up to 8 * NBL blocks): a lane's blocks are loaded before the
 // activation row is staged, one latency for both.
-template <int LAYOUT, bool REC, bool SHORT = false>
+template <int LAYOUT, bool REC, int NBL = 0>
 __global__ __launch_bounds__(256) void k_gemv_q4_grouped(GemvArgs a) {
     extern __shared__ int lds[];
     const int e = blockIdx.y;
@@ -309,13 +316,13 @@ __global__ __launch_bounds__(256) void k_gemv_q4_grouped(GemvArgs a) {
     const int sub = lane & 7;
     const bool live = row < a.n_rows;
     const uint8_t* wr = entry_base(a, e) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k);
-    Blocks4<LAYOUT> w4;
-    if constexpr (SHORT) w4.load(wr, sub, 8, nb, (nb * 2 + 15) / 16 * 16);
+    Blocks<LAYOUT, NBL ? NBL : 1> w4;
+    if constexpr (NBL > 0) w4.load(wr, sub, 8, nb, (nb * 2 + 15) / 16 * 16);
     stage_q8(a, e, lds);
     float acc = 0.0f;
     if (live) {
         int32_t* rec = REC ? a.dots + ((int64_t)e * a.n_rows + row) * nb : nullptr;
-        if constexpr (SHORT) acc = w4.template dots<REC>(0.0f, sub, 8, nb, lds, rec);
+        if constexpr (NBL > 0) acc = w4.template dots<REC>(0.0f, sub, 8, nb, lds, rec);
         else acc = gemv_row_part<LAYOUT, 8, REC>(wr, sub, nb, lds, rec);
     }
     acc = sum_row_lanes(acc);
@@ -583,10 +590,10 @@ __global__ __launch_bounds__(64 * LPR * WU, WU == 1 ? 24 / LPR : 1) void k_gemv_
 // + ...) for them, pairs in order. LPR lanes per row: 8 is
 // k_gemv_q4_grouped's arithmetic; 16 (long rows) sums each row's blocks in
 // 16 lane chains instead, twice the workgroups. Grid (ceil(H/R), n_seqs).
-// SHORT (rows of up to 4*LPR blocks): a lane's blocks are all loaded before the
-// activation rows are staged, one latency for both.
+// NBL > 0 (rows of up to NBL*LPR blocks): a lane's blocks are all loaded before
+// the activation rows are staged, one latency for both.
 // REC (test record): every int32 block dot also goes to a.dots[pair][row][block].
-template <int LAYOUT, int LPR, bool SHORT, bool REC>
+template <int LAYOUT, int LPR, int NBL, bool REC>
 __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const float* wts, const float* x, float* out,
                                                            int k) {
     extern __shared__ int lds[];
@@ -601,8 +608,8 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     const bool live = row < a.n_rows;
     // the row's address depends on a slot load: a long row's is formed after the staging, whose loads it would hold up
     auto wrow = [&] { return entry_base(a, s * k + kk) + (int64_t)(live ? row : 0) * row_bytes_of(LAYOUT, a.k); };
-    Blocks4<LAYOUT> w4;
-    if constexpr (SHORT) w4.load(wrow(), sub, LPR, nb, (nb * 2 + 15) / 16 * 16);  // the row's share, with the q8 rows
+    Blocks<LAYOUT, NBL ? NBL : 1> w4;
+    if constexpr (NBL > 0) w4.load(wrow(), sub, LPR, nb, (nb * 2 + 15) / 16 * 16);  // the row's share, with the q8 rows
     // up to 40 loads per thread in one batch: the k rows (36 words per thread
     // for two rows of 448 blocks) arrive in one load latency
     stage_words<40>(reinterpret_cast<const int*>(a.q8 + (int64_t)s * k * a.q8_stride_blocks * Q8_BLK), k * nb * 10,
@@ -610,7 +617,7 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     float acc = 0.0f;
     if (live) {
         int32_t* rec = REC && a.dots ? a.dots + ((int64_t)(s * k + kk) * a.n_rows + row) * nb : nullptr;
-        if constexpr (SHORT) acc = sub < nb ? w4.template dots<REC>(0.0f, sub, LPR, nb, lds + kk * nb * 10, rec) : 0.0f;
+        if constexpr (NBL > 0) acc = sub < nb ? w4.template dots<REC>(0.0f, sub, LPR, nb, lds + kk * nb * 10, rec) : 0.0f;
         else acc = gemv_row_part<LAYOUT, LPR, REC>(wrow(), sub, nb, lds + kk * nb * 10, rec);
     }
     acc = sum_row_lanes<LPR>(acc);
@@ -1793,6 +1800,18 @@ static void launch_short_f32in(bool rec, bool act, int nbl, dim3 grid, size_t ld
     else launch_short<LPR, 1, false>(rec, nbl, grid, lds, s, a);
 }
 
+// pick(N) with N the blocks of a lane of 8 where a row has up to 32 (they are
+// loaded before the activations, and no more than there are: loading four where
+// two are in the row costs 10 % in a long launch), else 0.
+template <typename F>
+static auto with_row_loads(int64_t nb, F pick) {
+    return nb <= 8 ? pick(std::integral_constant<int, 1>{})
+           : nb <= 16 ? pick(std::integral_constant<int, 2>{})
+           : nb <= 24 ? pick(std::integral_constant<int, 3>{})
+           : nb <= 32 ? pick(std::integral_constant<int, 4>{})
+                      : pick(std::integral_constant<int, 0>{});
+}
+
 static int gemv_common(ft_hip_ctx* ctx, void* stream, GemvArgs& a, int64_t n_entries, int64_t n_rows, int64_t k,
                        int layout, bool dots, const char* name) {
     if (k <= 0 || k % 32) return fail(FT_HIP_E_SHAPE, "%s: k=%lld must be a positive multiple of 32", name, (long long)k);
@@ -1831,13 +1850,12 @@ static int gemv_common(ft_hip_ctx* ctx, void* stream, GemvArgs& a, int64_t n_ent
         else launch_short<64>(rec, nbl, g2, lds, S(stream), a);
     } else {
         const bool q4r = layout == FT_LAYOUT_Q4R;
-        auto pick = [&](auto sh) {
-            constexpr bool SH = decltype(sh)::value;
-            return q4r ? (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4R, true, SH> : k_gemv_q4_grouped<FT_LAYOUT_Q4R, false, SH>)
-                       : (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4_0, true, SH> : k_gemv_q4_grouped<FT_LAYOUT_Q4_0, false, SH>);
-        };
-        hipLaunchKernelGGL(nb <= 32 ? pick(std::true_type{}) : pick(std::false_type{}), grid, dim3(256), lds, S(stream),
-                           a);
+        auto kern = with_row_loads(nb, [&](auto nbl) {
+            constexpr int N = decltype(nbl)::value;
+            return q4r ? (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4R, true, N> : k_gemv_q4_grouped<FT_LAYOUT_Q4R, false, N>)
+                       : (rec ? k_gemv_q4_grouped<FT_LAYOUT_Q4_0, true, N> : k_gemv_q4_grouped<FT_LAYOUT_Q4_0, false, N>);
+        });
+        hipLaunchKernelGGL(kern, grid, dim3(256), lds, S(stream), a);
     }
     return launch_status(name);
 }
@@ -2458,15 +2476,13 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
         const int R = (int)((l16 ? 16 : 32) / top_k);
         const dim3 g_dn((unsigned)((hidden + R - 1) / R), (unsigned)n_seqs);
         const bool q4r = layout == FT_LAYOUT_Q4R;
-        auto pick = [&](auto lpr, auto sh) {
-            constexpr int L = decltype(lpr)::value;
-            constexpr bool SH = decltype(sh)::value;
-            return q4r ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, L, SH, true> : k_gemv_down_combine<FT_LAYOUT_Q4R, L, SH, false>)
-                       : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, L, SH, true> : k_gemv_down_combine<FT_LAYOUT_Q4_0, L, SH, false>);
+        auto form = [&](auto lpr, auto nbl) {
+            constexpr int L = decltype(lpr)::value, N = decltype(nbl)::value;
+            return q4r ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, L, N, true> : k_gemv_down_combine<FT_LAYOUT_Q4R, L, N, false>)
+                       : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, true> : k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, false>);
         };
-        auto kern = l16 ? pick(std::integral_constant<int, 16>{}, std::false_type{})
-                    : inter / 32 <= 32 ? pick(std::integral_constant<int, 8>{}, std::true_type{})
-                                       : pick(std::integral_constant<int, 8>{}, std::false_type{});
+        auto kern = l16 ? form(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{})
+                        : with_row_loads(inter / 32, [&](auto nbl) { return form(std::integral_constant<int, 8>{}, nbl); });
         hipLaunchKernelGGL(kern, g_dn, dim3(256), l_dn, st, a, (const float*)wts, x, x_out, (int)top_k);
         return launch_status("moe_layer/down_combine");
     }

@@ -33,7 +33,8 @@ def test_gate_up_two_lanes_per_chain_same_bits(gemv, orc, hidden):
 
 
 @pytest.mark.parametrize("layout", [ft_hip.LAYOUT_Q4_0, ft_hip.LAYOUT_Q4R])
-@pytest.mark.parametrize("k,n_rows", [(64, 1), (992, 33), (1024, 31), (1056, 33)])
+@pytest.mark.parametrize("k,n_rows", [(64, 1), (992, 33), (1024, 31), (1056, 33), (256, 33), (288, 33), (512, 33),
+                                      (544, 33), (768, 33), (800, 33), (1280, 33), (1312, 33), (1792, 33), (1824, 33)])
 def test_gemv_rows_of_about_32_blocks(gemv, orc, layout, k, n_rows):
     ops.test_block_dots_and_gemv(gemv, orc, layout, k, n_rows)
 
