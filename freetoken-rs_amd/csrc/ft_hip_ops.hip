@@ -1805,7 +1805,8 @@ static void launch_short_f32in(bool rec, bool act, int nbl, dim3 grid, size_t ld
 // two are in the row costs 10 % in a long launch), else 0.
 template <typename F>
 static auto with_row_loads(int64_t nb, F pick) {
-    return nb <= 8 ? pick(std::integral_constant<int, 1>{})
+    return nb <= 0 ? pick(std::integral_constant<int, 0>{})
+           : nb <= 8 ? pick(std::integral_constant<int, 1>{})
            : nb <= 16 ? pick(std::integral_constant<int, 2>{})
            : nb <= 24 ? pick(std::integral_constant<int, 3>{})
            : nb <= 32 ? pick(std::integral_constant<int, 4>{})
@@ -2475,6 +2476,10 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
         const bool l16 = down_lanes(inter, top_k) == 16;
         const int R = (int)((l16 ? 16 : 32) / top_k);
         const dim3 g_dn((unsigned)((hidden + R - 1) / R), (unsigned)n_seqs);
+        // Rows of up to 32 blocks before the activations, while the launch is one round of three workgroups per CU:
+        // then the latency saved counts (Gemma shape, 1 token 6.9 -> 6.4 us); in longer launches other
+        // workgroups cover it, and the loads held up by the barrier cost (3 tokens 15.1 -> 16.6, 8 tokens 30 -> 33).
+        const bool early = (int64_t)g_dn.x * n_seqs <= 768;
         const bool q4r = layout == FT_LAYOUT_Q4R;
         auto form = [&](auto lpr, auto nbl) {
             constexpr int L = decltype(lpr)::value, N = decltype(nbl)::value;
@@ -2482,7 +2487,7 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
                        : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, true> : k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, false>);
         };
         auto kern = l16 ? form(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{})
-                        : with_row_loads(inter / 32, [&](auto nbl) { return form(std::integral_constant<int, 8>{}, nbl); });
+                        : with_row_loads(early ? inter / 32 : 0, [&](auto nbl) { return form(std::integral_constant<int, 8>{}, nbl); });
         hipLaunchKernelGGL(kern, g_dn, dim3(256), l_dn, st, a, (const float*)wts, x, x_out, (int)top_k);
         return launch_status("moe_layer/down_combine");
     }

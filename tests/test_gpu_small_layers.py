@@ -70,3 +70,29 @@ def test_reduce_pairs_rounds_bit_exact(gemv, orc, n_pairs, n_seqs, hidden):
 @pytest.mark.parametrize("hidden", [2816, 4096])
 def test_dot4_row_per_pair_matches_tiles(gemv, hidden, counts):
     tiles.test_token_tiles_match_dot4(gemv, hidden, 96, counts, True)
+
+
+@pytest.mark.parametrize("layout", [ft_hip.LAYOUT_Q4_0, ft_hip.LAYOUT_Q4R])
+@pytest.mark.parametrize("hidden,inter,n_experts,top_k,n", [(1024, 512, 8, 4, 16),   # many pairs per expert
+                                                            (2816, 704, 24, 8, 3),
+                                                            (3072, 768, 40, 4, 5)])
+def test_layer_of_many_tokens_same_bits_as_one_by_one(gemv, layout, hidden, inter, n_experts, top_k, n):
+    """A layer's forms go by the pairs and workgroups of the call: each token of
+    a batch has the bits of a call of its own."""
+    m = ops.moe_synth.SyntheticMoE(gemv, ops.moe_synth.Shape("small", hidden, inter, n_experts, top_k, 1, 9), n_layers=1,
+                                   layout=layout)
+    x = torch.stack([m.hidden(t) for t in range(n)])
+
+    def layer(part):
+        b = len(part)
+        ids = torch.zeros(b * top_k, dtype=torch.int32, device=DEV)
+        wts = torch.zeros(b * top_k, dtype=torch.float32, device=DEV)
+        out = torch.zeros_like(part)
+        m.layer(0, part, out, ids, wts, m.workspace(b), n_seqs=b)
+        return ops.host(out).view(np.uint32), ops.host(ids), ops.host(wts)
+
+    out, ids, wts = layer(x)
+    for t in range(n):
+        o, i, w = layer(x[t:t + 1].contiguous())
+        assert np.array_equal(o[0], out[t])
+        assert np.array_equal(i, ids[t * top_k:(t + 1) * top_k]) and np.array_equal(w, wts[t * top_k:(t + 1) * top_k])
