@@ -1764,21 +1764,32 @@ static void launch_gu_long(int bpl, dim3 grid, size_t lds, hipStream_t st, const
                                             wts, E, h);
 }
 
-// The gate|up launch with the activation, k_gemv_gu_act. q4r rows: two lanes
-// on each of a row's four chains (Gemma shape, gate|up launch: 12.1 us against
-// 13.0 for 1 token, 34.6 against 38.9 for 8; four lanes 12.3 and 59); q4_0
-// rows one (8 tokens 39.9 us against 42.4 with two).
+// The gate|up launch with the activation, k_gemv_gu_act. two: two lanes on each
+// of a row's four chains (two_lanes).
 template <bool TOPK, bool HEAD>
-static void launch_gu_act(int layout, bool rec, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a, int inter,
-                          uint8_t* q8a, const float* in_scale, int div, const float* logits, const float* escale,
-                          int32_t* ids, float* wts, int E, const HeadArgs& h) {
-    const bool q4r = layout == FT_LAYOUT_Q4R;
-    auto kern = q4r ? (rec ? k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, true, 2>
-                           : k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, false, 2>)
-                    : (rec ? k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, true>
-                           : k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, false>);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * GU_LANES * (q4r ? 2 : 1)), lds, st, a, inter, q8a, in_scale, div, logits,
+static void launch_gu_act(int layout, bool two, bool rec, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a,
+                          int inter, uint8_t* q8a, const float* in_scale, int div, const float* logits,
+                          const float* escale, int32_t* ids, float* wts, int E, const HeadArgs& h) {
+    auto kern = layout != FT_LAYOUT_Q4R ? (rec ? k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, true>
+                                               : k_gemv_gu_act<FT_LAYOUT_Q4_0, TOPK, GU_LANES, HEAD, false>)
+                : two ? (rec ? k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, true, 2>
+                             : k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, false, 2>)
+                      : (rec ? k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, true>
+                             : k_gemv_gu_act<FT_LAYOUT_Q4R, TOPK, GU_LANES, HEAD, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * GU_LANES * (two ? 2 : 1)), lds, st, a, inter, q8a, in_scale, div, logits,
                        escale, ids, wts, E, h);
+}
+
+// Two lanes on each chain of a gate|up row: for q4r rows of at least 32 blocks
+// whose weights come from memory, i.e. with no more pairs than experts (Gemma
+// shape, the launch: 12.2 -> 11.4 us for 1 token, 39.3 -> 36.2 for 8; layers of
+// 32 experts of hidden 1536 / 2560 / 5120: 2 tokens 17.3 -> 16.2 us, 20.3 -> 18.3,
+// 30.0 -> 26.1, 8 tokens 25.1 -> 24.3, 34.0 -> 33.6, 55.4 -> 54.2). Where pairs share them the dots
+// bound it and the handing over costs (16 tokens 35.6 -> 37.4, 50.0 -> 51.8, 85.2 -> 87.4; 64
+// tokens of hidden 1024 65 -> 80), and shorter rows leave its six rounds empty
+// (hidden 512, 1 token 13.8 -> 14.4). q4_0 rows: 8 tokens 39.9 -> 42.4.
+static bool two_lanes(int layout, int64_t hidden, int64_t n_pairs, int64_t n_experts) {
+    return layout == FT_LAYOUT_Q4R && hidden >= 32 * 32 && n_pairs <= n_experts;
 }
 
 template <int LPR, bool REC, int XIN = 0, bool ACT = false>
@@ -2135,7 +2146,9 @@ extern "C" int ft_hip_gemv_gate_up_act(ft_hip_ctx* ctx, void* stream, const void
                                      nullptr, nullptr, nullptr, nullptr, 0, HeadArgs{}, rec);
         return launch_status(nm);
     }
-    launch_gu_act<false, false>(layout, rec, grid, lds, S(stream), a, (int)inter, (uint8_t*)q8_act, in_scale,
+    // the bank's experts are not known here: short launches as pairs that share none
+    const bool two = two_lanes(layout, hidden, (int64_t)grid.x * grid.y, 768);
+    launch_gu_act<false, false>(layout, two, rec, grid, lds, S(stream), a, (int)inter, (uint8_t*)q8_act, in_scale,
                                 (int)x_div, nullptr, nullptr, nullptr, nullptr, 0, HeadArgs{});
     return launch_status(nm);
 }
@@ -2418,6 +2431,7 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
     const dim3 g_gu((unsigned)(inter / 32), (unsigned)n_pairs);
     const size_t l_gu = (size_t)(hidden / 32) * Q8_BLK;
     const int gbpl = gu_long_bpl(layout, hidden);
+    const bool two = two_lanes(layout, hidden, n_pairs, n_experts);
     a.sums = rec.gu;
     a.dots = rec.gu_dots;
     a.x8rec = rec.q8x;
@@ -2428,7 +2442,7 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
             launch_gu_long<true, true>(gbpl, g_gu, l_head, st, a, (int)inter, w.q8a, nullptr, (int)top_k, nullptr,
                                        expert_scale, ids, wts, (int)n_experts, h, rec.on);
         else
-            launch_gu_act<true, true>(layout, rec.on, g_gu, l_head, st, a, (int)inter, w.q8a, nullptr, (int)top_k,
+            launch_gu_act<true, true>(layout, two, rec.on, g_gu, l_head, st, a, (int)inter, w.q8a, nullptr, (int)top_k,
                                       nullptr, expert_scale, ids, wts, (int)n_experts, h);
     } else if (gbpl) {
         if (topk_in)
@@ -2438,10 +2452,10 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
             launch_gu_long<false, false>(gbpl, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
                                          expert_scale, ids, wts, (int)n_experts, HeadArgs{}, rec.on);
     } else if (topk_in) {
-        launch_gu_act<true, false>(layout, rec.on, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
+        launch_gu_act<true, false>(layout, two, rec.on, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
                                    expert_scale, ids, wts, (int)n_experts, HeadArgs{});
     } else {
-        launch_gu_act<false, false>(layout, rec.on, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
+        launch_gu_act<false, false>(layout, two, rec.on, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
                                     expert_scale, ids, wts, (int)n_experts, HeadArgs{});
     }
     if ((rc = launch_status("moe_layer/gate_up_act"))) return rc;

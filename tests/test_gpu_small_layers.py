@@ -1,6 +1,6 @@
 """The launches of small layers at the edges of their forms: the gate|up of
-q4r rows with two lanes on each of a row's chains (six rounds of eight blocks
-at once), the GEMV and down launches that load a row of up to 32 blocks before
+q4r rows of at least 32 blocks with two lanes on each of a row's chains (six
+rounds of eight blocks at once) while pairs share no weights, the GEMV and down launches that load a row of up to 32 blocks before
 the activations, the combine over a pair list in rounds of 256 pairs, and the
 dot4 layer with a workgroup row per pair (fewer pairs than experts)."""
 import numpy as np
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("hidden", [32, 160, 256, 1504, 1536, 1568, 2816, 3104])
+@pytest.mark.parametrize("hidden", [32, 160, 256, 992, 1024, 1056, 1504, 1536, 1568, 2816, 3104])
 def test_gate_up_two_lanes_per_chain_same_bits(gemv, orc, hidden):
     """q4_0 rows have one lane per chain: the same chains in the same order, so
     the act blocks of the two layouts are the same bytes."""
