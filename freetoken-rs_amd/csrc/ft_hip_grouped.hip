@@ -1105,9 +1105,10 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
 // block's activation operand); wave w works on K slice w (blocks [w*BW,
 // w*BW+BW) below nbj); the slice partials of a (row, token) are summed in
 // slice order into y[pair][row]. The partials overlay the tiles' scales in LDS
-// (restaged for each 16 tokens), so two workgroups fit a CU. Blocks go in NBB-block batches, NBUF batches in
-// flight (register buffers).
-template <int BW, int RT, int NBB, int NBUF, bool REC>
+// (restaged for each 16 tokens), so two workgroups fit a CU. Blocks go in
+// NBB-block batches, NBUF batches in flight (register buffers). ONCE: the rows
+// are loaded past the caches (nontemporal).
+template <int BW, int RT, int NBB, int NBUF, bool REC, bool ONCE>
 __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_t expert_bytes, int64_t gu_bytes,
                                                      const int32_t* meta, const int32_t* plist, const uint8_t* q8m,
                                                      int P, float* ydn, int H, int I, int E, int n_min,
@@ -1153,7 +1154,7 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
             if constexpr (NBB == 4) {
 #pragma unroll
                 for (int m = 0; m < RT; ++m) {
-                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, 2);
+                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, ONCE ? 2 : 0);
                     aw[buf][0][m] = v.x;
                     aw[buf][1][m] = v.y;
                     aw[buf][2][m] = v.z;
@@ -1491,8 +1492,17 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         } else {  // long rows: DRT tiles per workgroup, 8 K slices of 56 (rows up to 448 blocks) or 64 blocks
             constexpr int DRT = 4;
             const size_t lds_md = std::max((size_t)DRT * nbj * 32, sizeof(float) * GW * DRT * 16 * MT);
-            auto kern = nbj <= 8 * 56 ? (rec ? k_mfma_down<56, DRT, 4, 2, true> : k_mfma_down<56, DRT, 4, 2, false>)
-                                      : (rec ? k_mfma_down<64, DRT, 4, 2, true> : k_mfma_down<64, DRT, 4, 2, false>);
+            // The rows go past the caches while an expert's tokens mostly fit one tile of 16: past it they are read
+            // again (layer of the large-expert shape, 8 experts, past / through: 16 tokens 171.5 / 174.0 us, 32 178.6 /
+            // 180.5, 40 179.6 / 181.5, 48 234.5 / 236.6, 56 295 / 294, 64 296.8 / 295.5, 96 330.7 / 322.6).
+            const bool once = !rec && P <= 12 * E;
+            auto form = [&](auto on, auto rc) {
+                constexpr bool ON = decltype(on)::value, RC = decltype(rc)::value;
+                return nbj <= 8 * 56 ? k_mfma_down<56, DRT, 4, 2, RC, ON> : k_mfma_down<64, DRT, 4, 2, RC, ON>;
+            };
+            auto kern = once ? form(std::true_type{}, std::false_type{})
+                        : rec ? form(std::false_type{}, std::true_type{})
+                              : form(std::false_type{}, std::false_type{});
             hipLaunchKernelGGL(kern, dim3(H / (16 * DRT), gbig), dim3(GT), lds_md, s, (const uint8_t*)bank, eb,
                                gu_bytes, (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8m, P,
                                w.ydn, H, I, E, n_mfma, rdn);

@@ -52,11 +52,8 @@ __device__ __forceinline__ int entry_xrow(const GemvArgs& a, int e) {
     return a.x_idx ? a.x_idx[e] : e / a.x_div;
 }
 
-// 16 bytes of a weight row that no other load of the launch's lines follows
-// (nontemporal): for waves that read whole lines of rows of megabytes, where
-// the caches only cost. Large-expert shape, stack of one token and two layers
-// 93.3 -> 84.8 us with it on the gate|up and down rows; on short rows, whose lines
-// several loads share, it is slower (one token's Gemma-shaped layer 21.0 -> 23.6).
+// 16 bytes of a weight row, past the caches (nontemporal): for waves that read
+// whole lines of rows of megabytes in a launch that reads them once (read_once).
 __device__ __forceinline__ uint4 load_once(const uint8_t* p) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
@@ -212,7 +209,7 @@ struct Blocks {
 // together, the last one to four as well, no more than there are: a row is
 // otherwise one load latency per block). The caller sums the LPR lanes by xor
 // 1, 2, 4 (, 8).
-template <int LAYOUT, int LPR = 8, bool REC = false>
+template <int LAYOUT, int LPR = 8, bool REC = false, bool ONCE = false>
 __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int nb, const int* lds,
                                                int32_t* rec = nullptr) {
     const int qs_off = (nb * 2 + 15) / 16 * 16;
@@ -223,7 +220,7 @@ __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int n
         float d4[4];
         uint4 q[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) load_block<LAYOUT, (LPR > 8)>(wr, b + LPR * u, qs_off, d4[u], q[u]);
+        for (int u = 0; u < 4; ++u) load_block<LAYOUT, ONCE>(wr, b + LPR * u, qs_off, d4[u], q[u]);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int* xb = lds + (b + LPR * u) * 10;
@@ -248,7 +245,7 @@ __device__ __forceinline__ float gemv_row_part(const uint8_t* wr, int sub, int n
         for (; b < nb; b += LPR) {
             float d4;
             uint4 q;
-            load_block<LAYOUT, (LPR > 8)>(wr, b, qs_off, d4, q);
+            load_block<LAYOUT, ONCE>(wr, b, qs_off, d4, q);
             const int* xb = lds + b * 10;
             const float d8 = __int_as_float(xb[0]);
             const int diff = block_dot(q, xb + 2, xb[1]);
@@ -593,7 +590,7 @@ __global__ __launch_bounds__(64 * LPR * WU, WU == 1 ? 24 / LPR : 1) void k_gemv_
 // NBL > 0 (rows of up to NBL*LPR blocks): a lane's blocks are all loaded before
 // the activation rows are staged, one latency for both.
 // REC (test record): every int32 block dot also goes to a.dots[pair][row][block].
-template <int LAYOUT, int LPR, int NBL, bool REC>
+template <int LAYOUT, int LPR, int NBL, bool REC, bool ONCE = false>
 __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const float* wts, const float* x, float* out,
                                                            int k) {
     extern __shared__ int lds[];
@@ -618,7 +615,7 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
     if (live) {
         int32_t* rec = REC && a.dots ? a.dots + ((int64_t)(s * k + kk) * a.n_rows + row) * nb : nullptr;
         if constexpr (NBL > 0) acc = sub < nb ? w4.template dots<REC>(0.0f, sub, LPR, nb, lds + kk * nb * 10, rec) : 0.0f;
-        else acc = gemv_row_part<LAYOUT, LPR, REC>(wrow(), sub, nb, lds + kk * nb * 10, rec);
+        else acc = gemv_row_part<LAYOUT, LPR, REC, ONCE>(wrow(), sub, nb, lds + kk * nb * 10, rec);
     }
     acc = sum_row_lanes<LPR>(acc);
     if (sub == 0) ys[re] = acc;
@@ -643,7 +640,7 @@ __global__ __launch_bounds__(256) void k_gemv_down_combine(GemvArgs a, const flo
 // k_route_prep's chunk partials P_c, for head_prologue in the next gate|up
 // launch. Grid (H/16, n_seqs), NT = 16*k*LPR threads; E < NT.
 // REC (test record): every int32 block dot also goes to a.dots[pair][row][block].
-template <int LAYOUT, int LPR, int NT, bool REC = false>
+template <int LAYOUT, int LPR, int NT, bool REC, bool ONCE>
 __global__ __launch_bounds__(NT) void k_gemv_down_head(GemvArgs a, const float* wts, const float* x, float* out,
                                                       int k, const float* wnext, float* part, int E) {
     extern __shared__ int lds[];
@@ -680,7 +677,7 @@ __global__ __launch_bounds__(NT) void k_gemv_down_head(GemvArgs a, const float* 
     const int kk = re >> 4, rl = re & 15;
     const int row = c * 16 + rl;
     int32_t* rec = REC && a.dots ? a.dots + ((int64_t)(s * k + kk) * H + row) * nb : nullptr;
-    float acc = gemv_row_part<LAYOUT, LPR, REC>(entry_base(a, s * k + kk) + (int64_t)row * row_bytes_of(LAYOUT, a.k),
+    float acc = gemv_row_part<LAYOUT, LPR, REC, ONCE>(entry_base(a, s * k + kk) + (int64_t)row * row_bytes_of(LAYOUT, a.k),
                                                 sub, nb, lds + kk * nb * 10, rec);
     acc = sum_row_lanes<LPR>(acc);
     if (sub == 0) ys[re] = acc;
@@ -731,11 +728,14 @@ struct LongRow {
     uint32_t s[BPL];  // the aligned dword holding this lane's block scale and the neighbour lane's
 };
 
-template <int BPL>
+template <int BPL, bool ONCE>
 __device__ __forceinline__ void long_row_load(const uint8_t* wr, int lane, LongRow<BPL>& r) {
     constexpr int NB = 64 * BPL, QS_OFF = (NB * 2 + 15) / 16 * 16;
 #pragma unroll
-    for (int i = 0; i < BPL; ++i) r.q[i] = load_once(wr + QS_OFF + 16 * (lane + 64 * i));
+    for (int i = 0; i < BPL; ++i) {
+        const uint8_t* p = wr + QS_OFF + 16 * (lane + 64 * i);
+        r.q[i] = ONCE ? load_once(p) : *reinterpret_cast<const uint4*>(p);
+    }
 #pragma unroll
     for (int i = 0; i < BPL; ++i) r.s[i] = *reinterpret_cast<const uint32_t*>(wr + ((2 * (lane + 64 * i)) & ~3));
 }
@@ -781,7 +781,7 @@ __device__ __forceinline__ float long_row_dot(const LongRow<BPL>& r, const LongA
 // multiple of UPB) and the prologue is computed once for them; with UPB 1 the
 // grid is (inter/32, pairs). REC: the test record of k_gemv_gu_act (block
 // dots, sums, head q8 row).
-template <bool TOPK, int BPL, bool HEAD = false, bool REC = false, int UPB = 1>
+template <bool TOPK, int BPL, bool HEAD, bool REC, int UPB, bool ONCE>
 __global__ __launch_bounds__(256 * UPB, UPB == 1 ? 4 : 1) void k_gemv_gu_long(GemvArgs a, int inter, uint8_t* q8a,
                                                                              const float* in_scale, int div,
                                                                              const float* logits, const float* escale,
@@ -814,7 +814,7 @@ __global__ __launch_bounds__(256 * UPB, UPB == 1 ? 4 : 1) void k_gemv_gu_long(Ge
     const uint8_t* eb = nullptr;
     auto row_of = [&](int i) { return (i < 8 ? 0 : inter) + jb * 32 + 8 * wave + (i & 7); };
     auto load_row = [&](int i) __attribute__((always_inline)) {
-        long_row_load<BPL>(eb + (int64_t)row_of(i) * RB, lane, rr[i % RIF]);
+        long_row_load<BPL, ONCE>(eb + (int64_t)row_of(i) * RB, lane, rr[i % RIF]);
     };
     auto issue = [&](int slot) __attribute__((always_inline)) {
         eb = a.base + (uint64_t)slot * a.expert_bytes + a.bank_off;
@@ -1735,34 +1735,42 @@ static int gu_long_bpl(int layout, int64_t hidden) {
 // CU: the workgroups then spread evenly, 224 for the large-expert layer's
 // 896 units, instead of 3 or 4 of the 256-thread form per CU) when 4 divides
 // inter/32 and the layer has at least 128 such workgroups.
-template <bool TOPK, bool HEAD, bool REC = false>
+template <bool TOPK, bool HEAD, bool REC, bool ONCE>
 static void launch_gu_long_r(int bpl, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a, int inter,
                              uint8_t* q8a, const float* in_scale, int div, const float* logits, const float* escale,
                              int32_t* ids, float* wts, int E, const HeadArgs& h) {
     if (bpl == 2 && grid.x % 4 == 0 && grid.x * grid.y / 4 >= 128) {
-        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 2, HEAD, REC, 4>), dim3(grid.x * grid.y / 4), dim3(1024), lds, st, a,
-                           inter, q8a, in_scale, div, logits, escale, ids, wts, E, h);
+        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 2, HEAD, REC, 4, ONCE>), dim3(grid.x * grid.y / 4), dim3(1024), lds, st,
+                           a, inter, q8a, in_scale, div, logits, escale, ids, wts, E, h);
         return;
     }
     if (bpl == 1)
-        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 1, HEAD, REC>), grid, dim3(256), lds, st, a, inter, q8a, in_scale,
-                           div, logits, escale, ids, wts, E, h);
+        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 1, HEAD, REC, 1, ONCE>), grid, dim3(256), lds, st, a, inter, q8a,
+                           in_scale, div, logits, escale, ids, wts, E, h);
     else
-        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 2, HEAD, REC>), grid, dim3(256), lds, st, a, inter, q8a, in_scale,
-                           div, logits, escale, ids, wts, E, h);
+        hipLaunchKernelGGL((k_gemv_gu_long<TOPK, 2, HEAD, REC, 1, ONCE>), grid, dim3(256), lds, st, a, inter, q8a,
+                           in_scale, div, logits, escale, ids, wts, E, h);
 }
-// rec: the record instantiation (a layer record is set)
+// rec: the record instantiation (a layer record is set); once: read_once
 template <bool TOPK, bool HEAD>
 static void launch_gu_long(int bpl, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a, int inter, uint8_t* q8a,
                            const float* in_scale, int div, const float* logits, const float* escale, int32_t* ids,
-                           float* wts, int E, const HeadArgs& h, bool rec = false) {
-    if (rec)
-        launch_gu_long_r<TOPK, HEAD, true>(bpl, grid, lds, st, a, inter, q8a, in_scale, div, logits, escale, ids, wts,
-                                           E, h);
-    else
-        launch_gu_long_r<TOPK, HEAD, false>(bpl, grid, lds, st, a, inter, q8a, in_scale, div, logits, escale, ids,
-                                            wts, E, h);
+                           float* wts, int E, const HeadArgs& h, bool rec, bool once) {
+    auto launch = rec    ? launch_gu_long_r<TOPK, HEAD, true, false>
+                  : once ? launch_gu_long_r<TOPK, HEAD, false, true>
+                         : launch_gu_long_r<TOPK, HEAD, false, false>;
+    launch(bpl, grid, lds, st, a, inter, q8a, in_scale, div, logits, escale, ids, wts, E, h);
 }
+
+// Whether long weight rows (gate|up rows of 64 or 128 blocks, down rows of at
+// least 256) are loaded past the caches: as long as about no two pairs share an expert,
+// the caches only cost; from there on a row's second reader finds it in them.
+// Stacks of two large-expert layers (8 experts, top-2), past them / through
+// them: 1 token 86.6 / 95.0 us, 2 153 / 169, 4 289 / 296, 5 356 / 361, 6 418 / 415,
+// 8 524 / 515; a layer of hidden 2048, I 4096, 16 tokens 67 / 61, 64 tokens 205 /
+// 176. On shorter rows, whose lines several loads share, it is slower at any
+// number (one token's Gemma-shaped layer 21.0 -> 23.6).
+static bool read_once(int64_t n_pairs, int64_t n_experts) { return 4 * n_pairs <= 5 * n_experts; }
 
 // The gate|up launch with the activation, k_gemv_gu_act. two: two lanes on each
 // of a row's four chains (two_lanes).
@@ -2143,7 +2151,8 @@ extern "C" int ft_hip_gemv_gate_up_act(ft_hip_ctx* ctx, void* stream, const void
     const size_t lds = (size_t)(hidden / 32) * Q8_BLK;
     if (const int bpl = gu_long_bpl(layout, hidden)) {
         launch_gu_long<false, false>(bpl, grid, lds, S(stream), a, (int)inter, (uint8_t*)q8_act, in_scale, (int)x_div,
-                                     nullptr, nullptr, nullptr, nullptr, 0, HeadArgs{}, rec);
+                                     nullptr, nullptr, nullptr, nullptr, 0, HeadArgs{}, rec,
+                                     n_pairs <= x_div);  // one token's pairs: of distinct experts
         return launch_status(nm);
     }
     // the bank's experts are not known here: short launches as pairs that share none
@@ -2307,25 +2316,23 @@ static bool head_fold_ok(int64_t hidden, int64_t inter, int64_t n_experts, int64
 }
 
 // k_gemv_down_head for nt = 16*k*LPR threads (256, 512 or 1024)
-template <int LAYOUT, int LPR, bool REC>
+template <int LAYOUT, int LPR, bool REC, bool ONCE>
 static void launch_down_head_r(int nt, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a, const float* wts,
                                const float* x, float* out, int k, const float* wnext, float* part, int E) {
-    if (nt == 256)
-        hipLaunchKernelGGL((k_gemv_down_head<LAYOUT, LPR, 256, REC>), grid, dim3(256), lds, st, a, wts, x, out, k,
-                           wnext, part, E);
-    else if (nt == 512)
-        hipLaunchKernelGGL((k_gemv_down_head<LAYOUT, LPR, 512, REC>), grid, dim3(512), lds, st, a, wts, x, out, k,
-                           wnext, part, E);
-    else
-        hipLaunchKernelGGL((k_gemv_down_head<LAYOUT, LPR, 1024, REC>), grid, dim3(1024), lds, st, a, wts, x, out, k,
-                           wnext, part, E);
+    auto kern = nt == 256   ? k_gemv_down_head<LAYOUT, LPR, 256, REC, ONCE>
+                : nt == 512 ? k_gemv_down_head<LAYOUT, LPR, 512, REC, ONCE>
+                            : k_gemv_down_head<LAYOUT, LPR, 1024, REC, ONCE>;
+    hipLaunchKernelGGL(kern, grid, dim3(nt == 256 || nt == 512 ? nt : 1024), lds, st, a, wts, x, out, k, wnext, part, E);
 }
 template <int LAYOUT, int LPR>
-static void launch_down_head(bool rec, int nt, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a,
+static void launch_down_head(bool rec, bool once, int nt, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& a,
                              const float* wts, const float* x, float* out, int k, const float* wnext, float* part,
                              int E) {
-    if (rec) launch_down_head_r<LAYOUT, LPR, true>(nt, grid, lds, st, a, wts, x, out, k, wnext, part, E);
-    else launch_down_head_r<LAYOUT, LPR, false>(nt, grid, lds, st, a, wts, x, out, k, wnext, part, E);
+    constexpr bool LONG = LAYOUT == FT_LAYOUT_Q4R && LPR > 8;
+    auto launch = rec            ? launch_down_head_r<LAYOUT, LPR, true, false>
+                  : once && LONG ? launch_down_head_r<LAYOUT, LPR, false, LONG>
+                                 : launch_down_head_r<LAYOUT, LPR, false, false>;
+    launch(nt, grid, lds, st, a, wts, x, out, k, wnext, part, E);
 }
 
 // Test record of one layer of the launch-by-launch path (ft_hip_set_layer_record):
@@ -2431,7 +2438,7 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
     const dim3 g_gu((unsigned)(inter / 32), (unsigned)n_pairs);
     const size_t l_gu = (size_t)(hidden / 32) * Q8_BLK;
     const int gbpl = gu_long_bpl(layout, hidden);
-    const bool two = two_lanes(layout, hidden, n_pairs, n_experts);
+    const bool two = two_lanes(layout, hidden, n_pairs, n_experts), once = read_once(n_pairs, n_experts);
     a.sums = rec.gu;
     a.dots = rec.gu_dots;
     a.x8rec = rec.q8x;
@@ -2440,17 +2447,17 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
         const size_t l_head = l_gu + (size_t)(hidden / 16) * (n_experts + 1) * 4;
         if (gbpl)
             launch_gu_long<true, true>(gbpl, g_gu, l_head, st, a, (int)inter, w.q8a, nullptr, (int)top_k, nullptr,
-                                       expert_scale, ids, wts, (int)n_experts, h, rec.on);
+                                       expert_scale, ids, wts, (int)n_experts, h, rec.on, once);
         else
             launch_gu_act<true, true>(layout, two, rec.on, g_gu, l_head, st, a, (int)inter, w.q8a, nullptr, (int)top_k,
                                       nullptr, expert_scale, ids, wts, (int)n_experts, h);
     } else if (gbpl) {
         if (topk_in)
             launch_gu_long<true, false>(gbpl, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
-                                        expert_scale, ids, wts, (int)n_experts, HeadArgs{}, rec.on);
+                                        expert_scale, ids, wts, (int)n_experts, HeadArgs{}, rec.on, once);
         else
             launch_gu_long<false, false>(gbpl, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
-                                         expert_scale, ids, wts, (int)n_experts, HeadArgs{}, rec.on);
+                                         expert_scale, ids, wts, (int)n_experts, HeadArgs{}, rec.on, once);
     } else if (topk_in) {
         launch_gu_act<true, false>(layout, two, rec.on, g_gu, l_gu, st, a, (int)inter, w.q8a, inv, (int)top_k, w.logits,
                                    expert_scale, ids, wts, (int)n_experts, HeadArgs{});
@@ -2480,7 +2487,7 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
         auto launch = layout == FT_LAYOUT_Q4R
                           ? (lpr == 16 ? launch_down_head<FT_LAYOUT_Q4R, 16> : launch_down_head<FT_LAYOUT_Q4R, 8>)
                           : (lpr == 16 ? launch_down_head<FT_LAYOUT_Q4_0, 16> : launch_down_head<FT_LAYOUT_Q4_0, 8>);
-        launch(rec.on, nt, g_dn, l_dn, st, a, wts, x, x_out, (int)top_k, wnext, part_out, (int)n_experts);
+        launch(rec.on, once, nt, g_dn, l_dn, st, a, wts, x, x_out, (int)top_k, wnext, part_out, (int)n_experts);
         return launch_status("moe_layer/down_head");
     }
     if (32 % top_k == 0 && l_dn <= 64 * 1024) {
@@ -2500,7 +2507,8 @@ static int moe_layer_impl(const char* nm, ft_hip_ctx* ctx, void* stream, const f
             return q4r ? (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, L, N, true> : k_gemv_down_combine<FT_LAYOUT_Q4R, L, N, false>)
                        : (rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, true> : k_gemv_down_combine<FT_LAYOUT_Q4_0, L, N, false>);
         };
-        auto kern = l16 ? form(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{})
+        auto kern = l16 && q4r && once && !rec.on ? k_gemv_down_combine<FT_LAYOUT_Q4R, 16, 0, false, true>
+                    : l16 ? form(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{})
                         : with_row_loads(early ? inter / 32 : 0, [&](auto nbl) { return form(std::integral_constant<int, 8>{}, nbl); });
         hipLaunchKernelGGL(kern, g_dn, dim3(256), l_dn, st, a, (const float*)wts, x, x_out, (int)top_k);
         return launch_status("moe_layer/down_combine");

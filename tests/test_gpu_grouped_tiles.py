@@ -192,3 +192,33 @@ def test_tiles_found_without_the_grouping_launch(gemv, hidden, inter, E, K, B):
         torch.cuda.synchronize()
         got.append(out.cpu().numpy().view(np.uint32))
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("hidden,inter", [(2816, 1056), (4096, 14368)])
+def test_long_down_rows_same_bits_in_parts(gemv, hidden, inter):
+    """Rows of over 32 blocks, of experts with more than one tile of tokens (then
+    the rows are loaded through the caches) and with less."""
+    E, K, B = 2, 1, 40
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 82), ft_hip.LAYOUT_Q4R)
+    src = torch.empty(E * eb, dtype=torch.uint8, device=DEV)
+    for e in range(E):
+        gemv.gen_q4_rows(100 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(200 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    rng = np.random.default_rng(hidden)
+    x = torch.from_numpy(rng.standard_normal((B, hidden)).astype(np.float32)).to(DEV)
+    w = torch.from_numpy((rng.standard_normal((E, hidden)) * 0.02).astype(np.float32)).to(DEV)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+
+    def layer(part):
+        out = torch.zeros_like(part)
+        ids = torch.zeros(len(part) * K, dtype=torch.int32, device=DEV)
+        wts = torch.zeros(len(part) * K, dtype=torch.float32, device=DEV)
+        gemv.moe_layer_grouped(part, out, len(part), hidden, inter, E, K, w, None, None, bank, ids, wts, ws)
+        torch.cuda.synchronize()
+        return out.cpu().numpy().view(np.uint32)
+
+    out = layer(x)
+    for t0 in range(0, B, 20):  # 20 pairs: under 12 per expert
+        assert np.array_equal(layer(x[t0:t0 + 20].contiguous()), out[t0:t0 + 20])

@@ -1,8 +1,9 @@
 """The launches of small layers at the edges of their forms: the gate|up of
 q4r rows of at least 32 blocks with two lanes on each of a row's chains (six
-rounds of eight blocks at once) while pairs share no weights, the GEMV and down launches that load a row of up to 32 blocks before
-the activations, the combine over a pair list in rounds of 256 pairs, and the
-dot4 layer with a workgroup row per pair (fewer pairs than experts)."""
+rounds of eight blocks at once) while pairs share no weights, the GEMV and down
+launches that load a row of up to 32 blocks before the activations, the combine
+over a pair list in rounds of 256 pairs, and the dot4 layer with a workgroup
+row per pair (fewer pairs than experts)."""
 import numpy as np
 import pytest
 import torch
@@ -75,7 +76,8 @@ def test_dot4_row_per_pair_matches_tiles(gemv, hidden, counts):
 @pytest.mark.parametrize("layout", [ft_hip.LAYOUT_Q4_0, ft_hip.LAYOUT_Q4R])
 @pytest.mark.parametrize("hidden,inter,n_experts,top_k,n", [(1024, 512, 8, 4, 16),   # many pairs per expert
                                                             (2816, 704, 24, 8, 3),
-                                                            (3072, 768, 40, 4, 5)])
+                                                            (3072, 768, 40, 4, 5),
+                                                            (2048, 8192, 8, 2, 6)])      # long rows, read more than once
 def test_layer_of_many_tokens_same_bits_as_one_by_one(gemv, layout, hidden, inter, n_experts, top_k, n):
     """A layer's forms go by the pairs and workgroups of the call: each token of
     a batch has the bits of a call of its own."""
