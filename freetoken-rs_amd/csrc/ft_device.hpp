@@ -245,15 +245,6 @@ __device__ __forceinline__ void quad_transpose(uint32_t& a0, uint32_t& a1, uint3
     a3 = s3[1];
 }
 
-__device__ __forceinline__ void quad_transpose_f(float& a0, float& a1, float& a2, float& a3) {
-    uint32_t u0 = __float_as_uint(a0), u1 = __float_as_uint(a1), u2 = __float_as_uint(a2), u3 = __float_as_uint(a3);
-    quad_transpose(u0, u1, u2, u3);
-    a0 = __uint_as_float(u0);
-    a1 = __uint_as_float(u1);
-    a2 = __uint_as_float(u2);
-    a3 = __uint_as_float(u3);
-}
-
 // ---------------------------------------------------------------------------
 // GELU and the softmax exp with the bits of the libm calls ft-core makes
 // (f32::tanh, ft-model/src/lib.rs:436; f32::exp, :1495): restatements of

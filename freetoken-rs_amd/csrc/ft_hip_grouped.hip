@@ -537,9 +537,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ uint32_t buf_ld(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-}
 
 // A token's q8 block as the B operand of lane group g, from the q8m layout
 // (GroupWs::q8m): q8 words (g, g+4) at vq + sq, {d, qsum} at vd + sd, one
@@ -1106,19 +1103,17 @@ __global__ __launch_bounds__(NW * 64, LANES ? 3 : 4) void k_mfma_down_tok(
 // w*BW+BW) below nbj); the slice partials of a (row, token) are summed in
 // slice order into y[pair][row]. The partials overlay the tiles' scales in LDS
 // (restaged for each 16 tokens), so two workgroups fit a CU. Blocks go in
-// NBB-block batches, NBUF batches in flight (register buffers). ONCE: the rows
-// are loaded past the caches (nontemporal).
-template <int BW, int RT, int NBB, int NBUF, bool REC, bool ONCE>
+// batches of four, NBUF batches in flight (register buffers). ONCE: the rows are
+// loaded past the caches (nontemporal).
+template <int BW, int RT, int NBUF, bool REC, bool ONCE>
 __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_t expert_bytes, int64_t gu_bytes,
                                                      const int32_t* meta, const int32_t* plist, const uint8_t* q8m,
-                                                     int P, float* ydn, int H, int I, int E, int n_min,
-                                                     int32_t* rec) {
+                                                     int P, float* ydn, int H, int I, int E, int32_t* rec) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int nbj = I >> 5, dn_tile = nbj * 288;
     const int u = blockIdx.x, g = blockIdx.y;
-    if (g >= meta[1 + 3 * E]) return;  // groups of >= n_min tokens come first
+    if (g >= meta[1 + 3 * E]) return;
     const int e = meta[1 + g], s0 = meta[1 + E + g], n = meta[1 + 2 * E + g];
-    if (n < n_min) return;
     // LDS: the tiles' scales [RT][nbj][16] f16; slice partials [GW][RT][16][MT]
     // in the same bytes once the K loop is done
     uint16_t* scl = reinterpret_cast<uint16_t*>(lds);
@@ -1130,7 +1125,7 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
     // the RT tiles: qs of tile tile0+m at m*dn_tile + nbj*32 from D0 + tile0*dn_tile
     const __amdgpu_buffer_rsrc_t rw = buf_rsrc(D0 + (int64_t)tile0 * dn_tile, (uint32_t)(RT * dn_tile));
     const __amdgpu_buffer_rsrc_t ra = buf_rsrc(q8m, (uint32_t)P * nbj * Q8_BLK);  // < NO_TOKEN bytes
-    const uint32_t vw = nbj * 32 + li * 16 + 4 * lg, vw4 = nbj * 32 + lg * 256 + li * 16;
+    const uint32_t vw4 = nbj * 32 + lg * 256 + li * 16;
     for (int c0 = 0; c0 < n; c0 += MT) {
         const int nt = min(MT, n - c0);
         const int q = s0 + c0 + min(li, nt - 1), p = plist[q];
@@ -1140,34 +1135,28 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
         const bool ok = li < nt;
         const uint32_t vq = ok ? (uint32_t)(lg * P + q) * 8 : NO_TOKEN;
         const uint32_t vd = ok ? (uint32_t)P * nbj * 32 + (uint32_t)q * 8 : NO_TOKEN;
-        // blocks in NBB-block batches, the loads of the batch NBUF - 1 ahead
+        // blocks in batches of four, the loads of the batch NBUF - 1 ahead
         // issued before the current batch's MFMAs (NBUF register buffers)
-        constexpr int NBATCH = BW / NBB;
+        constexpr int NBB = 4, NBATCH = BW / NBB;
         uint32_t aw[NBUF][NBB][RT];
         ActOp av[NBUF][NBB];
-        // NBB == 4: one 16-byte load per tile for the batch's four blocks,
+        // one 16-byte load per tile for the batch's four blocks,
         // lane group g taking all four qs words of its row in block 4k+g (1 KB
         // contiguous per wave), turned into word g of each block by
         // quad_transpose when the batch is consumed (blocks past the row are
         // read, never used: the descriptor bounds the reads)
         auto load = [&](int k, int buf) __attribute__((always_inline)) {
-            if constexpr (NBB == 4) {
 #pragma unroll
-                for (int m = 0; m < RT; ++m) {
-                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, ONCE ? 2 : 0);
-                    aw[buf][0][m] = v.x;
-                    aw[buf][1][m] = v.y;
-                    aw[buf][2][m] = v.z;
-                    aw[buf][3][m] = v.w;
-                }
+            for (int m = 0; m < RT; ++m) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, ONCE ? 2 : 0);
+                aw[buf][0][m] = v.x;
+                aw[buf][1][m] = v.y;
+                aw[buf][2][m] = v.z;
+                aw[buf][3][m] = v.w;
             }
 #pragma unroll
             for (int b = 0; b < NBB; ++b) {
                 const int bb = min(bs + k * NBB + b, nbj - 1);
-                if constexpr (NBB != 4) {
-#pragma unroll
-                    for (int m = 0; m < RT; ++m) aw[buf][b][m] = buf_ld(rw, vw, m * dn_tile + bb * 256);
-                }
                 av[buf][b] = act_op_m(ra, vq, vd, bb * 32 * P, bb * 8 * P);
             }
         };
@@ -1202,10 +1191,8 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
             // wait below counts only this batch's loads, not the prefetch's
             load(k + NBUF - 1, (j + NBUF - 1) % NBUF);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (NBB == 4) {
 #pragma unroll
-                for (int m = 0; m < RT; ++m) quad_transpose(aw[j][0][m], aw[j][1][m], aw[j][2][m], aw[j][3][m]);
-            }
+            for (int m = 0; m < RT; ++m) quad_transpose(aw[j][0][m], aw[j][1][m], aw[j][2][m], aw[j][3][m]);
 #pragma unroll
             for (int b = 0; b < NBB; ++b) {
                 if (bs + k * NBB + b < nbj) {  // uniform
@@ -1498,14 +1485,14 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
             const bool once = !rec && P <= 12 * E;
             auto form = [&](auto on, auto rc) {
                 constexpr bool ON = decltype(on)::value, RC = decltype(rc)::value;
-                return nbj <= 8 * 56 ? k_mfma_down<56, DRT, 4, 2, RC, ON> : k_mfma_down<64, DRT, 4, 2, RC, ON>;
+                return nbj <= 8 * 56 ? k_mfma_down<56, DRT, 2, RC, ON> : k_mfma_down<64, DRT, 2, RC, ON>;
             };
             auto kern = once ? form(std::true_type{}, std::false_type{})
                         : rec ? form(std::false_type{}, std::true_type{})
                               : form(std::false_type{}, std::false_type{});
             hipLaunchKernelGGL(kern, dim3(H / (16 * DRT), gbig), dim3(GT), lds_md, s, (const uint8_t*)bank, eb,
                                gu_bytes, (const int32_t*)w.meta, (const int32_t*)w.plist, (const uint8_t*)w.q8m, P,
-                               w.ydn, H, I, E, n_mfma, rdn);
+                               w.ydn, H, I, E, rdn);
         }
         if ((rc = launch_status("moe_layer_grouped/down_mfma"))) return rc;
     }
