@@ -1125,7 +1125,12 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
     // the RT tiles: qs of tile tile0+m at m*dn_tile + nbj*32 from D0 + tile0*dn_tile
     const __amdgpu_buffer_rsrc_t rw = buf_rsrc(D0 + (int64_t)tile0 * dn_tile, (uint32_t)(RT * dn_tile));
     const __amdgpu_buffer_rsrc_t ra = buf_rsrc(q8m, (uint32_t)P * nbj * Q8_BLK);  // < NO_TOKEN bytes
+    constexpr int NBB = 4, NBATCH = BW / NBB;
+    // this slice's batches (uniform; none when the slice starts past nbj)
+    const int nbat = max(0, min(NBATCH, (nbj - bs + NBB - 1) / NBB));
+    // this lane's row and block in a batch, and in the slice's last one
     const uint32_t vw4 = nbj * 32 + lg * 256 + li * 16;
+    const uint32_t vwl = nbj * 32 + min(lg, nbj - 1 - (bs + (nbat - 1) * NBB)) * 256 + li * 16;
     for (int c0 = 0; c0 < n; c0 += MT) {
         const int nt = min(MT, n - c0);
         const int q = s0 + c0 + min(li, nt - 1), p = plist[q];
@@ -1137,18 +1142,21 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
         const uint32_t vd = ok ? (uint32_t)P * nbj * 32 + (uint32_t)q * 8 : NO_TOKEN;
         // blocks in batches of four, the loads of the batch NBUF - 1 ahead
         // issued before the current batch's MFMAs (NBUF register buffers)
-        constexpr int NBB = 4, NBATCH = BW / NBB;
         uint32_t aw[NBUF][NBB][RT];
         ActOp av[NBUF][NBB];
         // one 16-byte load per tile for the batch's four blocks,
         // lane group g taking all four qs words of its row in block 4k+g (1 KB
         // contiguous per wave), turned into word g of each block by
-        // quad_transpose when the batch is consumed (blocks past the row are
-        // read, never used: the descriptor bounds the reads)
+        // quad_transpose when the batch is consumed (past the slice its last
+        // batch again, past the row its last block, never used: no read leans on
+        // the descriptor's range check, which may not see the scalar offset)
         auto load = [&](int k, int buf) __attribute__((always_inline)) {
+            const int kw = min(k, nbat - 1);  // uniform
+            const uint32_t vw = kw < nbat - 1 ? vw4 : vwl;
 #pragma unroll
             for (int m = 0; m < RT; ++m) {
-                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, vw4, m * dn_tile + (bs + k * 4) * 256, ONCE ? 2 : 0);
+                const u32x4 v =
+                    __builtin_amdgcn_raw_buffer_load_b128(rw, vw, m * dn_tile + (bs + kw * NBB) * 256, ONCE ? 2 : 0);
                 aw[buf][0][m] = v.x;
                 aw[buf][1][m] = v.y;
                 aw[buf][2][m] = v.z;
@@ -1165,8 +1173,6 @@ __global__ __launch_bounds__(GT, 4) void k_mfma_down(const uint8_t* bank, int64_
         for (int m = 0; m < RT; ++m)
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[m][v] = 0.0f;
-        // this slice's batches (uniform; none when the slice starts past nbj)
-        const int nbat = max(0, min(NBATCH, (nbj - bs + NBB - 1) / NBB));
 #pragma unroll
         for (int k = 0; k < NBUF - 1; ++k)
             if (k < nbat) load(k, k);
