@@ -59,8 +59,11 @@ def check_pair(orc, rec_gu, rec_dn, gu_rows, dn_rows, x, act_blk, where):
     assert np.array_equal(rec_dn, orc.block_dots(dn_rows, aq, aq.size)), f"down {where}"
 
 
-@pytest.mark.parametrize("shape,B,mfma_min,norm", [("gemma", 16, 0, False),       # dot4, 1 pair per expert
+@pytest.mark.parametrize("shape,B,mfma_min,norm", [("gemma", 16, 10 ** 6, False),  # dot4, 1 pair per expert
                                                    ("gemma", 64, 10 ** 6, True),  # dot4, ~4 pairs per expert
+                                                   ("gemma", 5, 0, False),        # dot4, a workgroup row per pair
+                                                   ("gemma", 10, 0, True),        # the last batch of the automatic dot4
+                                                   ("gemma", 11, 0, True),        # the first of its MFMA tiles
                                                    ("gemma", 16, 1, False),       # int8 MFMA tiles
                                                    ("large", 3, 0, False)])       # MFMA, K-split long down rows
 def test_grouped_block_dots_bit_exact(gemv, orc, shape, B, mfma_min, norm):

@@ -10,8 +10,9 @@ The ungrouped launch-by-launch layer (one GEMV per pair, as the reference's
 batched path, ft-model/src/lib.rs:1507-1606) must pick the same experts with
 the same weights. With the input RMS norm on, its scale enters the logits
 and the gate|up sums; the same checks hold. The default (mfma_min 0) puts every
-expert on the int8 MFMA tile kernels from 2/3 of a pair per expert on (B = 16,
-64, 128) and on the dot4 kernels below (mfma_min 10**6 forces them); cases also split the experts at 16 tokens
+expert on the int8 MFMA tile kernels from 2/3 of a pair per expert on (B = 11,
+16, 64, 128) and on the dot4 kernels below (B = 5 and 10: fewer pairs than
+experts, a workgroup row per pair); cases also split the experts at 16 tokens
 (both families in one layer) and force every expert onto one family (mfma_min
 1 or 10**6); the large-expert shape (inter 14336) always takes the MFMA
 kernels.
@@ -53,6 +54,8 @@ def _banks(m, layer, ids):
 
 
 @pytest.mark.parametrize("B,zipf,norm,mfma_min", [(16, False, False, 0), (64, False, False, 0), (128, False, False, 0),
+                                                   (16, False, False, 10**6), (5, False, True, 0),
+                                                   (10, False, False, 0), (10, False, True, 0), (11, False, True, 0),
                                                    (64, True, False, 16),
                                                   (16, True, True, 16), (16, False, False, 1), (64, True, True, 1),
                                                   (64, True, False, 10**6)])
