@@ -7,7 +7,9 @@
 // gemv_q4r_ptr, reduce_pairs_weighted), re-reading an expert's weights for
 // every token routed to it. Here:
 //   router logits + top-k + q8(x)         (the launch-by-launch kernels)
-//   k_group_pairs     one workgroup: pairs per expert, active-expert list
+//   k_group_pairs     one workgroup: pairs per expert, active-expert list (not in
+//                     layers of up to 512 pairs on one family: their workgroups
+//                     find their pairs in the routing)
 //   k_grouped_gu      per (active expert, gate|up tile j): the tile's 64 rows
 //                     in registers, dots against every token of the expert,
 //                     GELU*up, q8 of the act block -> act[pair][j]
@@ -273,10 +275,10 @@ __device__ __forceinline__ int scan_pairs(const int32_t* ids, int P, int e, int*
 // Gate|up tile j of active expert g for all of its tokens, then GELU*up and
 // the q8 of act block j per token. BPW = H/32/8 blocks per wave. in_scale
 // (input RMS norm, or null): a token's gate|up sums are first multiplied by
-// in_scale[token]. SCAN: the grid's y is the expert, or a pair
-// if there are fewer of those (empty workgroups: 2,046 of 2,816 at 5 tokens of
-// the Gemma shape, now 110 of 880), and the workgroup finds its expert's pairs
-// in ids[0..P) (scan_pairs) instead of the group list.
+// in_scale[token]. SCAN: the grid's y is the expert, or a pair if there are
+// fewer of those (5 tokens of the Gemma shape: 110 of 880 workgroups find
+// nothing to do, of one row per expert 2,046 of 2,816), and the workgroup finds
+// its expert's pairs in ids[0..P) (scan_pairs) instead of the group list.
 template <int BPW, bool REC, bool SCAN>
 __global__ __launch_bounds__(GT, 2) void k_grouped_gu(const uint8_t* bank, int64_t expert_bytes, const int32_t* meta,
                                                       const int32_t* plist, const uint8_t* q8x, uint8_t* q8a,
@@ -672,9 +674,10 @@ struct TileScan {
     }
 };
 
-// Gate|up of the MFMA groups by token tiles: workgroup (x, y) takes act blocks
-// x*NW .. x*NW + NW-1 (one wave each: the 64 rows of tile j) for tile y of the
-// token tiles that k_group_pairs lists (up to 16*TT tokens of one expert).
+// Gate|up of the MFMA groups by token tiles (up to 16 tokens of one expert): a
+// workgroup takes one tile (of k_group_pairs' list, or with SCAN found by its
+// waves) and NW consecutive act blocks j, one wave each (the 64 rows of gate|up
+// tile j); the grid is one-dimensional over these units.
 // The tokens' q8 rows are staged in LDS once, by block, so that a lane's
 // operand words are one 8-byte read; a wave streams its tile's rows through a
 // register ring of one K slice (BPW blocks, 1 KB per load), its scales
@@ -691,10 +694,11 @@ struct TileScan {
 // tile of a group of over 16 tokens, on ranges of tiles that skewed token
 // counts left uneven: 475 us for 512 tokens of the Gemma shape and 855 us for
 // 173 zipf-skewed ones. Here a wave needs no other wave: 118-126 and 67 us.
-// What bounds it: for many tokens the VALU (72 % busy: 16 conversions and 16
-// fmas per block and wave are left after the scale products moved to the
-// matrix cores, 24 for operands and 10 for the GELU epilogue); for few the
-// weights (64 tokens: 285 MB in 63 us, 4.5 TB/s). Blocks are consumed one at a
+// What bounds it: for many tokens the VALU (512 tokens: 63 instructions per
+// block and wave, 71 % of the SIMDs' cycles, the matrix cores 24 %: 16
+// conversions and 16 fmas are left after the scale products moved to the
+// matrix cores, the others prepare operands or are the GELU epilogue); for few
+// the weights (64 tokens: 285 MB in 63 us, 4.5 TB/s; the VALU 53 %). Blocks are consumed one at a
 // time (sched_barrier), else the registers of a whole slice's dots spill.
 // KS, for launches of few units: a workgroup is one act block, its 8 waves a
 // slice each, and the first adds their sums in slice order, the same bits. The
@@ -948,10 +952,10 @@ __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
 // (row, token) acc = fma(float(D_b), d4_b * d8_b, acc) in block order, or with
 // LANES k_grouped_down's sums, bit for bit: four chains of blocks 4k, 4k + 1, ...,
 // products rounded before they are added, the chains as (0 + 1) + (2 + 3). Its
-// 48 registers more leave three waves a SIMD, and a layer of 11 to 63 tokens of the
-// Gemma shape takes 0.8 to 1.8 us longer (uniform routing 16 tokens 85.8 us against
-// 84.9, 63 tokens 120.3 against 118.5). Four
-// waves of about 94 registers per workgroup, several to a CU, so that one's
+// 48 registers more leave three waves a SIMD, and a layer of 11 to 63 tokens of
+// the Gemma shape takes 0.8 to 1.8 us longer (uniform routing 16 tokens 85.8 us
+// against 84.9, 63 tokens 120.3 against 118.5).
+// Four waves of about 94 registers per workgroup, several to a CU, so that one's
 // staging runs under another's dots (8 waves 64 us against 57 at 512 tokens;
 // two batches ahead instead of one 58.5). Before, one workgroup walked all of
 // an expert's tokens, rereading the weights for each 16: 512 tokens of the
@@ -1415,7 +1419,7 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
         };
         // Three forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
         // for all 128 of the Gemma shape), and small workgroups that hold half of the tokens' rows at a time
-        // (36 KB of LDS, 3 to a CU) spread them best over the CUs: 64 tokens 63 us against 73 for the other
+        // (31 KB of LDS; their 165 registers let 3 on a CU) spread them best over the CUs: 64 tokens 63 us against 73 for the other
         // form, 127 tokens 64 against 73 (zipf-skewed 55 against 65). More tokens: the VALU bounds it, and 8
         // waves share one staging of whole rows, two workgroups to a CU: 512 tokens 118-126 us against 137,
         // 173 zipf-skewed tokens 67 against 70; at 10 pairs per expert 74 against 80 (zipf-skewed 67, 71).
