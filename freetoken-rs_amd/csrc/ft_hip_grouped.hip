@@ -703,7 +703,7 @@ struct TileScan {
 // KS, for launches of few units: a workgroup is one act block, its 8 waves a
 // slice each, and the first adds their sums in slice order, the same bits. The
 // chain of a wave is an eighth as long: 16 tokens over 8 experts of H 4096, I 1024
-// 104 -> 41 us a layer, of H 2816, I 704 45 -> 34.
+// 104 -> 41 us a layer (against the 16-wave form), of H 2816, I 704 45 -> 34.
 template <int BPW, int NW, int WPE, int D, int KH, bool REC, bool SCAN, bool KS>
 __global__ __launch_bounds__(NW * 64, WPE) void k_mfma_gu_tok(
     const uint8_t* __restrict__ bank, int64_t expert_bytes, const int32_t* __restrict__ meta, uint32_t* tiles,
@@ -1359,9 +1359,9 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // tokens 119 / 86 against 160 / 252: dot4's cost grows with an expert's tokens),
     // and, below 4, only from 64 pairs (H 2816) or 96 (H 4096) on: fewer leave the
     // MFMA kernels' larger units too few (32 experts of I 704: 48 pairs 50 / 47 against
-    // 47 / 54, 64 pairs 50 / 48 against 52 / 62; 64 experts of H 4096, I 1024: 64 pairs
-    // 112 / 106 against 98 / 90, 96 pairs 120 / 112 against 118 / 115, 128 pairs 124 /
-    // 115 against 135 / 136)
+    // 47 / 54, 64 pairs 50 / 48 against 52 / 62; 32 experts of H 4096, I 1024, K-split
+    // form: 48 pairs 85 / 72 against 77 / 74, 64 88 / 76 against 86 / 88, 96 90 / 84
+    // against 101 / 111)
     int n_mfma = ctx->grouped_mfma_min;
     const bool sparse = P < 4LL * n_experts;
     if (n_mfma <= 0)
@@ -1417,20 +1417,24 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
                                (const int32_t*)w.plist, (const uint8_t*)w.q8x, w.q8m, dbg_gu, inv, I, E, K, P, rgu,
                                (const int32_t*)ids, (uint32_t*)w.q8a);
         };
-        // Three forms of one kernel. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
+        // Forms of one kernel. H 2816. Few tokens per expert: the weights bound it (one tile per expert, 285 MB
         // for all 128 of the Gemma shape), and small workgroups that hold half of the tokens' rows at a time
         // (31 KB of LDS; their 165 registers let 3 on a CU) spread them best over the CUs: 64 tokens 63 us against 73 for the other
         // form, 127 tokens 64 against 73 (zipf-skewed 55 against 65). More tokens: the VALU bounds it, and 8
         // waves share one staging of whole rows, two workgroups to a CU: 512 tokens 118-126 us against 137,
         // 173 zipf-skewed tokens 67 against 70; at 10 pairs per expert 74 against 80 (zipf-skewed 67, 71).
         // Few (tile, act block) units for the chip's 256 CUs: a wave that walks whole rows takes 25 us (H 2816) or
-        // 80 (H 4096, 16 to a CU) however few they are, so the 8 slices of a row go to 8 waves. Layers, that form
-        // against the other, uniform / zipf-skewed routing, by this bound on the units: H 2816 (I 704) 550 units 43 /
-        // 43 us against 58 / 59, 704 (under 9 pairs per expert) 42 / 39 against 47 / 46, 792 53 / 42 against 50 / 48,
-        // 902 58 / 56 against 55 / 56, 1056 (over) 64 / 64 against 67 / 67, 1760 94 / 95 against 80 / 81; H 4096
-        // (I 1024) 768 73 against 113, 1536 100 / 111 against 119 / 123, 2048 149 / 164 against 128 / 131.
+        // 35 to 80 (H 4096, 4 to 16 waves a CU) however few they are, so the 8 slices of a row go to 8 waves. Layers,
+        // that form against the other, uniform / zipf-skewed routing, by this bound on the units: H 2816 (I 704) 550
+        // units 43 / 43 us against 58 / 59, 704 (under 9 pairs per expert) 42 / 39 against 47 / 46, 792 53 / 42 against
+        // 50 / 48, 902 58 / 56 against 55 / 56, 1056 (over) 64 / 64 against 67 / 67, 1760 94 / 95 against 80 / 81; H
+        // 4096 (I 1024) 512 53 against 62, 704 58 / 61 against 61 / 63, 768 72 against 69, 1024 80 against 71.
+        // H 4096 has two forms more, by the units too: the 4 waves with half of the rows spread few units over more
+        // CUs, the 16 of one CU read the rows in larger pieces (the large-expert shape): 1312 units 70 / 73 us
+        // against 114, 2624 115 / 103 against 137 / 132, 3072 124 / 128 against 142 / 139, 3584 148 / 141 against 143
+        // / 139, 4032 186 / 180 against 167 / 160.
         const int64_t units = (int64_t)nbj * n_tiles;
-        const bool ks = !rec && units <= (H == 2816 ? (P < 9 * E ? 3 : 4) : 6) * 256;
+        const bool ks = !rec && units <= (H == 2816 && P >= 9 * E ? 4 : 3) * 256;
         if (H == 2816 && ks)
             gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, true>
                           : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false, true>, 8, 1, 1);
@@ -1445,6 +1449,9 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
             gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, false>
                     : rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false, false>
                           : k_mfma_gu_tok<11, 8, 4, 6, 1, false, false, false>, 8, 1, 8);
+        else if (!rec && units <= 12 * 256)
+            gate_up(tscan ? k_mfma_gu_tok<16, 4, 3, 5, 2, false, true, false>
+                          : k_mfma_gu_tok<16, 4, 3, 5, 2, false, false, false>, 4, 2, 4);
         else
             gate_up(tscan ? k_mfma_gu_tok<16, 16, 4, 6, 1, false, true, false>
                     : rec ? k_mfma_gu_tok<16, 16, 4, 6, 1, true, false, false>

@@ -27,7 +27,8 @@ DEV = "cuda:0"
     # (these few units take the form of a slice per wave; enough of them for the forms of an act block per wave)
     (2816, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 1] * 9 + [7]),          # 4 waves
     (2816, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 17] * 9 + [16]),        # 8: over 9 pairs per expert
-    (4096, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 4, 3, 1] * 8 + [48]),   # 16
+    (4096, 992, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 4, 3, 1] * 8 + [48]),   # 4, of H 4096
+    (4096, 1024, [1, 15, 16, 17, 0, 33, 0, 2] + [0, 4, 3, 1] * 22 + [48]),  # 16
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_token_tiles_match_dot4(gemv, hidden, inter, counts, norm):
@@ -166,7 +167,7 @@ def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, 
         gemv.set_grouped_mfma_min(0)
 
 
-@pytest.mark.parametrize("hidden,inter,E,K,B", [(2816, 992, 40, 8, 48), (2816, 96, 40, 8, 48), (4096, 992, 40, 4, 100),
+@pytest.mark.parametrize("hidden,inter,E,K,B", [(2816, 992, 40, 8, 48), (2816, 96, 40, 8, 48), (4096, 992, 40, 4, 100), (4096, 1024, 100, 4, 120),
                                                 (4096, 96, 40, 4, 41), (2816, 992, 100, 4, 128)])
 def test_tiles_found_without_the_grouping_launch(gemv, hidden, inter, E, K, B):
     """A call that asks for the act blocks goes through the grouping launch; the
