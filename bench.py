@@ -77,7 +77,7 @@ def parse():
                          "shape at batch 1")
     ap.add_argument("--mfma-min", type=int, default=0,
                     help="grouped path: experts with at least this many tokens take the int8 MFMA kernels "
-                         "(0: automatic, every expert on MFMA from 2/3 of a pair per expert and 64 (hidden 4096: 96) pairs on)")
+                         "(0: automatic, every expert on MFMA from 2/3 of a pair per expert and 64 (hidden 4096: 96, small layers: 40) pairs on)")
     ap.add_argument("--gemv-lanes", type=int, choices=[0, 8, 16, 32, 64], default=0,
                     help="dense config: lanes per row of the q4r GEMV launches (0: automatic)")
     ap.add_argument("--layers", type=int, default=0, help="0 = the config's layer count")

@@ -1361,11 +1361,17 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
     // MFMA kernels' larger units too few (32 experts of I 704: 48 pairs 50 / 47 against
     // 47 / 54, 64 pairs 50 / 48 against 52 / 62; 32 experts of H 4096, I 1024, K-split
     // form: 48 pairs 85 / 72 against 77 / 74, 64 88 / 76 against 86 / 88, 96 90 / 84
-    // against 101 / 111)
+    // against 101 / 111); from 40 in layers of up to two units of the K-split gate|up
+    // per CU (16 experts of I 704: 48 pairs 40 / 39 against 45 / 51; 32 experts, 748
+    // units, 40 pairs 48 against 44)
     int n_mfma = ctx->grouped_mfma_min;
     const bool sparse = P < 4LL * n_experts;
-    if (n_mfma <= 0)
-        n_mfma = sparse && (3LL * P < 2 * n_experts || P < (H == 2816 ? 64 : 96)) ? std::numeric_limits<int>::max() : 1;
+    // (tile, act block) units of the MFMA gate|up with every group on it, at most
+    const int64_t all_units = (int64_t)nbj * std::min(P, P / MT + std::min(E, P));
+    if (n_mfma <= 0) {
+        const int few = all_units <= 2 * 256 ? 40 : H == 2816 ? 64 : 96;
+        n_mfma = sparse && (3LL * P < 2 * n_experts || P < few) ? std::numeric_limits<int>::max() : 1;
+    }
     if (nbj > 32) n_mfma = 1;
     // Automatic, below 4 pairs per expert: the down sums in the dot4 kernels' order, so that where the line above
     // lies in this range shows in no output bit (another order of 22 block sums moves q8 quants of the layers that

@@ -401,7 +401,7 @@ class Q4Gemv:
 
     def set_grouped_mfma_min(self, n_tokens):
         """moe_layer_grouped: experts with >= n_tokens tokens take the MFMA kernels (0, the default:
-        all MFMA from 2/3 of a pair per expert and 64 (hidden 4096: 96) pairs on, else all dot4)."""
+        all MFMA from 2/3 of a pair per expert and 64 (hidden 4096: 96, small layers: 40) pairs on, else all dot4)."""
         check(lib().ft_hip_set_grouped_mfma_min(self._ctx, int(n_tokens)))
 
     def stream_read(self, buf, out, n_workgroups, nbytes=None, stream=None):

@@ -381,8 +381,8 @@ int ft_hip_moe_stack_grouped(ft_hip_ctx* ctx, void* stream, const float* x_in, f
  * block dots, routing and GELU q8 are the same). 0 (the default) = automatic:
  * every expert on the MFMA kernels when the batch has at least 2/3 of a (token,
  * expert) pair per expert (3 * n_seqs * top_k >= 2 * n_experts) and 64 pairs in
- * all (hidden 4096: 96), or 4 pairs per expert; else every expert on the dot4
- * kernels. Below 4 pairs per expert the output bits are the same on either
+ * all (hidden 4096: 96; small layers: 40), or 4 pairs per expert; else every
+ * expert on the dot4 kernels. Below 4 pairs per expert the output bits are the same on either
  * family. 1 = MFMA for every expert. Rows longer than 1024 weights (inter > 1024) always take
  * the MFMA kernels. No reference counterpart (the reference runs one GEMV
  * per (token, expert) pair, ft-model/src/lib.rs:1507-1606). */

@@ -132,6 +132,8 @@ def test_routing_of_many_seqs_matches_few(gemv, hidden, E, K, B, norm):
     (2816, 96, 257, 8, 64),    # more experts
     (4096, 96, 200, 3, 171),   # more pairs
     (2816, 96, 40, 4, 30),
+    (2816, 704, 16, 4, 10),    # 40 pairs: the first batch on the K-split form
+    (4096, 512, 16, 4, 10),
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_automatic_family_keeps_the_bits_under_4_pairs_per_expert(gemv, hidden, inter, E, K, B, norm):
