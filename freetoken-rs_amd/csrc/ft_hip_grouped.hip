@@ -1448,9 +1448,9 @@ extern "C" int ft_hip_moe_layer_grouped(ft_hip_ctx* ctx, void* stream, const flo
             gate_up(tscan ? k_mfma_gu_tok<16, 8, 2, 16, 1, false, true, true>
                           : k_mfma_gu_tok<16, 8, 2, 16, 1, false, false, true>, 8, 1, 1);
         else if (H == 2816 && P < 9 * E)
-            gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 8, 2, false, true, false>
+            gate_up(tscan ? k_mfma_gu_tok<11, 4, 3, 5, 2, false, true, false>
                     : rec ? k_mfma_gu_tok<11, 4, 3, 8, 2, true, false, false>
-                          : k_mfma_gu_tok<11, 4, 3, 7, 2, false, false, false>, 4, 2, 4);
+                          : k_mfma_gu_tok<11, 4, 3, 5, 2, false, false, false>, 4, 2, 4);
         else if (H == 2816)
             gate_up(tscan ? k_mfma_gu_tok<11, 8, 4, 6, 1, false, true, false>
                     : rec ? k_mfma_gu_tok<11, 8, 4, 6, 1, true, false, false>
