@@ -192,35 +192,31 @@ __global__ __launch_bounds__(1024) void k_group_pairs(const int32_t* ids, int P,
     // 1024): within each wavefront by shuffles, then each thread adds the
     // totals of the wavefronts before its own (integer sums: exact in any order)
     const int c = t < E ? cnt[t] : 0;
-    int vc = c, va = c > 0, vf = c > 0 && c >= n_mfma;
-    const int my_tiles = vf ? (c + MT - 1) / MT : 0;
-    int vt = my_tiles;
+    const bool vbig = c > 0 && c >= n_mfma;
+    const int my_tiles = vbig ? (c + MT - 1) / MT : 0;
+    // two sums to a word: pairs (up to 4096, 13 bits) and active experts, MFMA groups (up to 1024, 11 bits) and tiles
+    int s0 = c | (c > 0) << 13, s1 = (int)vbig | my_tiles << 11;
     const int lane = t & 63, wv = t >> 6;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const int nc = __shfl_up(vc, d), na = __shfl_up(va, d), nf = __shfl_up(vf, d), ntl = __shfl_up(vt, d);
+        const int n0 = __shfl_up(s0, d), n1 = __shfl_up(s1, d);
         if (lane >= d) {
-            vc += nc;
-            va += na;
-            vf += nf;
-            vt += ntl;
+            s0 += n0;
+            s1 += n1;
         }
     }
-    __shared__ int wtot[4][16];
+    __shared__ int wtot[2][16];
     __shared__ int n_tiles;
     if (lane == 63) {
-        wtot[0][wv] = vc;
-        wtot[1][wv] = va;
-        wtot[2][wv] = vf;
-        wtot[3][wv] = vt;
+        wtot[0][wv] = s0;
+        wtot[1][wv] = s1;
     }
     __syncthreads();
     for (int q = 0; q < wv; ++q) {
-        vc += wtot[0][q];
-        va += wtot[1][q];
-        vf += wtot[2][q];
-        vt += wtot[3][q];
+        s0 += wtot[0][q];
+        s1 += wtot[1][q];
     }
+    const int vc = s0 & 0x1FFF, va = s0 >> 13, vf = s1 & 0x7FF, vt = s1 >> 11;
     if (t == 1023) n_tiles = vt;
     scan[t] = vc;
     act[t] = va;
