@@ -41,9 +41,9 @@ HBM_PEAK_GBPS = 8000.0
 MEASURED_TRAFFIC = {
     "gemma30": 883615384,    # k_moe_stack_fused, one launch (algorithmic 846,151,680 B)
     "zipf": 888320417,       # k_moe_stack_fused, one launch
-    "batch16": 7637684432,   # whole step, 30 grouped layers (MFMA)
-    "batch64": 12071897377,  # whole step, 30 grouped layers (MFMA)
-    "large32": 25492686456,  # whole step, 32 grouped layers (MFMA)
+    "batch16": 7636078318,   # whole step, 30 grouped layers (MFMA)
+    "batch64": 12071680051,  # whole step, 30 grouped layers (MFMA)
+    "large32": 25492627526,  # whole step, 32 grouped layers (MFMA)
     "large1": 132272406,     # k_gemv_gu_long, one launch (algorithmic 132,120,576 B)
 }
 METRIC = "MoE expert-FFN µs/token at batch 1 + achieved HBM GB/s (% of MI355X peak)"

@@ -694,7 +694,7 @@ struct TileScan {
 // block and wave, 71 % of the SIMDs' cycles, the matrix cores 24 %: 16
 // conversions and 16 fmas are left after the scale products moved to the
 // matrix cores, the others prepare operands or are the GELU epilogue); for few
-// the weights (64 tokens: 285 MB in 63 us, 4.5 TB/s; the VALU 53 %). Blocks are consumed one at a
+// the weights (64 tokens: 285 MB in 63 us, 4.5 TB/s; the VALU 52 %). Blocks are consumed one at a
 // time (sched_barrier), else the registers of a whole slice's dots spill.
 // KS, for launches of few units: a workgroup is one act block, its 8 waves a
 // slice each, and the first adds their sums in slice order, the same bits. The
