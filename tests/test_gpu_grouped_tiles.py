@@ -225,3 +225,42 @@ def test_long_down_rows_same_bits_in_parts(gemv, hidden, inter):
     out = layer(x)
     for t0 in range(0, B, 20):  # 20 pairs: under 12 per expert
         assert np.array_equal(layer(x[t0:t0 + 20].contiguous()), out[t0:t0 + 20])
+
+
+@pytest.mark.parametrize("hidden,inter,E,K,B", [(2816, 704, 64, 8, 20), (4096, 96, 40, 4, 41)])
+def test_captured_layer_replays(gemv, hidden, inter, E, K, B):
+    """A layer whose workgroups find their tiles, captured once: every replay on
+    new inputs, with other work between, has the bits of the call itself."""
+    gu_b, _, eb = moe_synth.expert_geometry(moe_synth.Shape("t", hidden, inter, E, K, 1, 83), ft_hip.LAYOUT_Q4R)
+    src = torch.empty(E * eb, dtype=torch.uint8, device=DEV)
+    for e in range(E):
+        gemv.gen_q4_rows(300 + e, 0, 2 * inter, hidden, moe_synth.gen_scale(0.02), src[e * eb:e * eb + gu_b])
+        gemv.gen_q4_rows(400 + e, 0, hidden, inter, moe_synth.gen_scale(0.02), src[e * eb + gu_b:(e + 1) * eb])
+    bank = torch.empty(E * gemv.fused_expert_bytes(hidden, inter), dtype=torch.uint8, device=DEV)
+    gemv.pack_experts_fused(src, ft_hip.LAYOUT_Q4R, eb, bank, E, hidden, inter)
+    rng = np.random.default_rng(hidden)
+    xs = [torch.from_numpy(rng.standard_normal((B, hidden)).astype(np.float32)).to(DEV) for _ in range(4)]
+    w = torch.from_numpy((rng.standard_normal((E, hidden)) * 0.02).astype(np.float32)).to(DEV)
+    x, out = xs[0].clone(), torch.zeros_like(xs[0])
+    ids = torch.zeros(B * K, dtype=torch.int32, device=DEV)
+    wts = torch.zeros(B * K, dtype=torch.float32, device=DEV)
+    ws = torch.empty(gemv.moe_layer_grouped_workspace_bytes(B, hidden, inter, E, K), dtype=torch.uint8, device=DEV)
+
+    def layer():
+        gemv.moe_layer_grouped(x, out, B, hidden, inter, E, K, w, None, None, bank, ids, wts, ws)
+
+    want = []
+    for v in xs:
+        x.copy_(v)
+        layer()
+        torch.cuda.synchronize()
+        want.append(out.cpu().numpy().view(np.uint32))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer()
+    for v, exp in list(zip(xs, want)) * 2:
+        x.copy_(v)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), exp)
